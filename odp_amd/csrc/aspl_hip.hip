@@ -39,7 +39,13 @@ static const int RES_WB_MAX = 8;                // widest resident block: 256 so
 static const int BATCH_CLASSES = 5;             // size classes of the batch launch policy
 static const int FRONTIER_MIN_LEVELS = 16;      // frontier-mode levels when the last evaluation needed more
 static const u32 LIST_CAP = 1u << 22;           // unsaturated chunks a level may list (32 MiB)
+static const int LIST_COUNTERS = 2 * LIST_SUBS * LIST_PAD;   // the counters of two lists
+static const u32 THIN_CAP = 1u << 20;           // chunks a thin level may list (24 MiB),
+static const u32 THIN2_CAP = 1u << 18;          // ... and k_thin leave unsaturated
+static const double THIN_LEFT = 1.0 / 256;      // share of the chunks the thin neighbours should leave unsaturated
+static const double THIN2_READS = 8e6;          // chunk reads k_thin2 may take (two steps from every chunk left)
 static const double LIST_MAX_FRAC = 1.0 / 8;     // ... listed only when at most this share was left last time
+static const double LIST_MAX_FRAC_PG = 1.0 / 32; // ... by k_pgather, whose count-only levels cost less
 static const int LV_MISS_LEVELS = 64;            // levels whose missing pairs an evaluation records
 // adjacency tables up to this size reach the device through the resident
 // plan's table build reading pinned host memory (one kernel instead of a DMA
@@ -249,11 +255,41 @@ static int pg_aux_env()
 
 // the share of unsaturated chunks up to which a count-only last level lists
 // them (env ODP_HIP_LIST_FRAC; a large value always lists)
-static double list_frac_env()
+// ODP_HIP_FOLD=0: every unit of a gather level, whatever the table (diagnostics)
+static bool pg_fold_env()
+{
+  const char* v = getenv("ODP_HIP_FOLD");
+  return !v || atoi(v) != 0;
+}
+
+// ODP_HIP_THIN=0: no thin levels (diagnostics)
+static bool pg_thin_env()
+{
+  const char* v = getenv("ODP_HIP_THIN");
+  return !v || atoi(v) != 0;
+}
+
+// log2 of the pieces the units of k_pgather's last, partly filled round are cut
+// into: `units` of an XCD's workgroups in rounds of `wgs`, `extra` more at the
+// end.  A piece costs its share of a unit and about an eighth of one more (the
+// fill of its gathers, its barriers).
+static int pg_cut(double units, double extra, int wgs)
+{
+  const double rest = units - wgs * std::floor(units / wgs) + extra;
+  int best = 0;
+  double cost = 1e30;
+  for (int c = 0; c <= PG_CUT_MAX; c++) {
+    const double v = std::ceil(rest * (1 << c) / wgs - 1e-9) * (1.0 / (1 << c) + (c ? 0.125 : 0));
+    if (v < cost - 1e-9) { cost = v; best = c; }
+  }
+  return best;
+}
+
+static double list_frac_env(double dflt)
 {
   const char* v = getenv("ODP_HIP_LIST_FRAC");
-  const double f = v ? atof(v) : LIST_MAX_FRAC;
-  return f >= 0 ? f : LIST_MAX_FRAC;
+  const double f = v ? atof(v) : dflt;
+  return f >= 0 ? f : dflt;
 }
 
 // capacity of the unsaturated-chunk list (env ODP_HIP_LIST_CAP lowers it; the
@@ -329,12 +365,19 @@ struct LevelRun {
   u32* tq = nullptr;                    // k_tile's unit list (tile mode): lengths, queue head, entries
   size_t tq_cap = 0;
   u64* list = nullptr;                  // unsaturated chunks of the level before a count-only one
-  u32* list_n = nullptr;
+  u32* list_n = nullptr;                // the two lists' counters (after the done flags)
+  u32* asym = nullptr;                  // set unless the table is symmetric (after them)
   u32 list_cap = 0;
+  // thin levels (k_thin): the chunks of a list with their bits, and the second list
+  int thin = 0;                         // neighbours the pair lists mark thin
+  u64x2* list_v = nullptr;
+  u64* list2 = nullptr; u64x2* list2_v = nullptr;
   u64* h_acnt = nullptr;                // processed-unit counts on the host (kernel timing only)
   size_t flag_bytes = 0;
   // part-phased gather (k_pgather): row parts, sorted neighbour runs, persistent grid
   int parts = 0, psp = 0, pgrid = 0, pupt = 0, paux = 0;
+  bool fold = false;                    // folded levels where the table is symmetric (k_pgather)
+  int cut_full = 0, cut_fold = 0;       // log2 of the pieces its last round's units are cut into
   u32* plist = nullptr; int* ppoff = nullptr;  // per unit of PG_UNIT rows: pairs grouped by part, offsets
   size_t plist_cap = 0, ppoff_cap = 0;
   LevelTask* tasks = nullptr; int* wg_start = nullptr;
@@ -394,6 +437,10 @@ struct Evaluator {
   // the level plan's pair lists (k_plist) match its table (device swaps rebuild
   // the units of the rows they change); meaningful while table_fresh holds
   bool pl_fresh = false;
+  // the level plan's asymmetry flag (after the done flags) is the current
+  // table's: set by its check, outlived by device swaps (a swap of a symmetric
+  // table leaves it symmetric) while table_fresh holds
+  bool asym_fresh = false;
   // a batch of levels ends with k_lvfin: counters and error flag in host memory,
   // then its sequence number (lvseq: the last one enqueued; d_lvseq: the device's)
   LvHost* lvh = nullptr;
@@ -472,7 +519,7 @@ struct Evaluator {
         for (int i = 0; i < units.cnt; i++) seen = seen || units.u[i] == u;
         if (!seen) units.u[units.cnt++] = u;
       }
-      pl.nbr = d_nbr; pl.n = n; pl.dpad = dpad; pl.sp = lr.psp; pl.P = lr.parts; pl.list = lr.plist; pl.poff = lr.ppoff;
+      pl.nbr = d_nbr; pl.n = n; pl.dpad = dpad; pl.sp = lr.psp; pl.P = lr.parts; pl.thin = lr.thin; pl.list = lr.plist; pl.poff = lr.ppoff;
     }
     if (!mv.cnt && !units.cnt) return;
     auto kern = dpad + 1 <= 20 ? k_swap_at<20> : dpad + 1 <= 36 ? k_swap_at<36> : k_swap_at<64>;
@@ -488,6 +535,7 @@ struct Evaluator {
   void swap_launch(int a, int b, int c, int d, const int* pos = nullptr)
   {
     const SwapTables tb = patch_tables();
+    if (has_numdeg) asym_fresh = false;    // an entry past num_degrees may change in the adjacency alone
     const int rows[4] = {a, b, c, d}, from[4] = {b, a, d, c}, to[4] = {c, d, a, b};
     PlMove mv{};
     if (pos) {
@@ -509,6 +557,9 @@ struct Evaluator {
   // list_frac_env(), or after a dense one at most half that (no flip-flop of the
   // captured launch sequence between evaluations of similar graphs)
   bool list_on = true;
+  // neighbours a thin level takes (0: the last level's predecessor runs whole),
+  // from the last evaluation's reached pairs
+  int thin_k = 0;
   int batch_cap = MAX_BATCH_LEVELS;     // gather levels launched between two host reads (serving: few)
   hipStream_t st = nullptr;             // launch stream (the library's main stream unless set)
   bool timed() const { return g_stats_on && st == C.stream; }
@@ -516,9 +567,9 @@ struct Evaluator {
   // hipGraph of one evaluation's launch sequence: replayed while the plan, the
   // buffers, the adjacency pointer and (level plan) the first batch are unchanged
   hipGraphExec_t gexec = nullptr;
-  int g_key = -1;
+  long long g_key = -1;
   const int* g_adj = nullptr;
-  int g_seen = -1;                      // key of the last eager evaluation, for the repeat test
+  long long g_seen = -1;                      // key of the last eager evaluation, for the repeat test
   const int* g_seen_adj = nullptr;
   void drop_graph()
   {
@@ -532,11 +583,11 @@ struct Evaluator {
   // serving engine's slots (their own streams) launch eagerly.
   bool graph_on() const { return graphs_env() && !timed() && st == C.stream; }
   const int* cur_adj() const { return ext_adj ? ext_adj : d_adj; }
-  bool graph_ready(int key) const { return gexec && g_key == key && g_adj == cur_adj(); }
+  bool graph_ready(long long key) const { return gexec && g_key == key && g_adj == cur_adj(); }
   // Replay a graph only for a launch sequence that repeats: the first evaluation
   // of a key runs eagerly, the second captures, later ones replay.  One-off
   // evaluations (a new shape or plan every call) never pay for a capture.
-  bool use_graph(int key)
+  bool use_graph(long long key)
   {
     if (!graph_on()) return false;
     if (graph_ready(key) || (g_seen == key && g_seen_adj == cur_adj())) return true;
@@ -544,7 +595,7 @@ struct Evaluator {
     g_seen_adj = cur_adj();
     return false;
   }
-  template <typename F> void capture(F enqueue, int key)
+  template <typename F> void capture(F enqueue, long long key)
   {
     drop_graph();
     hipGraph_t g;
@@ -575,7 +626,8 @@ struct Evaluator {
     dfree(&lr.bufs); dfree(&lr.cnt); dfree(&lr.done); dfree(&lr.tasks); dfree(&lr.wg_start); hfree(&lr.h_cnt);
     lr.h_cnt_dev = nullptr;
     hfree(&lvh); lvh_dev = nullptr; dfree(&d_lvseq); lvseq = 0;
-    dfree(&lr.flags); hfree(&lr.h_acnt); dfree(&lr.wgm); dfree(&lr.list); dfree(&lr.list_n); dfree(&lr.tq);
+    dfree(&lr.flags); hfree(&lr.h_acnt); dfree(&lr.wgm); dfree(&lr.list); dfree(&lr.tq);
+    dfree(&lr.list_v); dfree(&lr.list2); dfree(&lr.list2_v);
     dfree(&lr.plist); dfree(&lr.ppoff);
     dfree(&rr.tasks); dfree(&rr.out); dfree(&rr.qhead); dfree(&rr.done); hfree(&rr.host); rr.host_dev = nullptr;
     dfree(&rr.part); rr.part_cap = 0;
@@ -583,7 +635,7 @@ struct Evaluator {
     bfs_q_cap = bfs_vis_cap = 0; bfs = false;
     lr = LevelRun(); rr = ResRun();
     adj_cap = nbr_cap = stage_cap = 0;
-    guess_levels = 0; list_on = true;
+    guess_levels = 0; list_on = true; thin_k = 0;
   }
 
   // shape of the graph; (re)allocates the graph buffers when they grow
@@ -677,6 +729,21 @@ struct Evaluator {
     return lm;
   }
 
+  // the change takes and adds as many entries u of row r as entries r of row u:
+  // it leaves a symmetric table symmetric (and is checked on the device otherwise)
+  static bool symmetric_change(const PlMove& mv)
+  {
+    auto delta = [&](int r, int u) {
+      int c = 0;
+      for (int e = 0; e < mv.cnt; e++) if (mv.row[e] == r) c += (mv.to[e] == u) - (mv.from[e] == u);
+      return c;
+    };
+    for (int e = 0; e < mv.cnt; e++)
+      for (int u : {mv.from[e], mv.to[e]})
+        if (u != mv.row[e] && delta(mv.row[e], u) != delta(u, mv.row[e])) return false;
+    return true;
+  }
+
   // a few changed entries against the last upload (at most RES_PATCH_MAX, of a
   // regular s = 1 table, every new id valid) under the resident plan with its
   // table current: queue them for the next launch (which stores them into the
@@ -713,6 +780,7 @@ struct Evaluator {
         h_stage[i] = a[i];
       }
       mv.cnt = k;
+      if (!symmetric_change(mv)) asym_fresh = false;
       entries_launch(patch_tables(), mv, rows, k);
     } else {
       for (int q = 0; q < k; q++) {
@@ -929,7 +997,8 @@ struct Evaluator {
     if ((size_t)ntasks > r.task_cap) {
       dfree(&r.cnt); dfree(&r.done); dfree(&r.tasks); dfree(&r.wg_start); hfree(&r.h_cnt);
       dalloc(&r.cnt, (size_t)3 * RING * ntasks);     // counts, changed, processed
-      dalloc(&r.done, (size_t)ntasks + 1);          // done flags, then the table's asymmetry flag
+      // done flags, the lists' counters (all cleared by the preparation), the table's asymmetry flag
+      dalloc(&r.done, (size_t)ntasks + LIST_COUNTERS + 1);
       hfree(&r.h_acnt); halloc(&r.h_acnt, (size_t)RING * ntasks);
       dalloc(&r.tasks, (size_t)ntasks); dalloc(&r.wg_start, (size_t)ntasks + 1);
       halloc_coherent(&r.h_cnt, &r.h_cnt_dev, (size_t)RING * ntasks);
@@ -940,7 +1009,9 @@ struct Evaluator {
     r.upw = plan.upw; r.seg_major = plan.seg_major; r.xcd = plan.xcd; r.urow = (lpr_log2 == 6);
     r.batch = plan.batch == 8 || plan.batch == 16 ? plan.batch : 4;
     r.per_task_wg = (units + 4 * r.upw - 1) / (4 * r.upw);
-    if (!r.list) { dalloc(&r.list, (size_t)LIST_CAP); dalloc(&r.list_n, (size_t)LIST_SUBS * LIST_PAD); }
+    if (!r.list) dalloc(&r.list, (size_t)LIST_CAP);
+    r.list_n = r.done + ntasks;
+    r.asym = r.list_n + LIST_COUNTERS;
     r.list_cap = (list_cap_env() + LIST_SUBS - 1) / LIST_SUBS;        // per sub-list
     if (plan.tile && tile_capable()) {
       const size_t cap = 3 + (size_t)group * ((width + TILE_MIN - 1) / TILE_MIN) * ((height + TILE_MIN - 1) / TILE_MIN);
@@ -954,21 +1025,33 @@ struct Evaluator {
     // the XCD-phased gather applies to 16-word rows and runs of at most 63 ids
     // the XCD-phased gather applies to 16-word rows, runs of at most 63 ids and
     // ids below 2^22 (the pair lists pack the row in the unit beside the id)
+    r.fold = false;
     r.parts = (plan.parts > 0 && kwp == 16 && dpad + 1 <= 63 && n <= (1 << 22)) ? plan.parts : 0;
     plan.parts = r.parts;              // the plan reports what runs
     if (r.parts) {
       r.psp = round_up(dpad + 1, 4);
       r.pupt = (n + PG_UNIT - 1) / PG_UNIT;
-      const size_t nl = (size_t)r.pupt * PG_UNIT * r.psp, np = (size_t)r.pupt * (PG_MAXP + 1);
+      const size_t nl = (size_t)r.pupt * PG_UNIT * r.psp, np = (size_t)r.pupt * PG_OFF;
       if (nl > r.plist_cap) { dfree(&r.plist); dalloc(&r.plist, nl); r.plist_cap = nl; }
       if (np > r.ppoff_cap) { dfree(&r.ppoff); dalloc(&r.ppoff, np); r.ppoff_cap = np; }
       r.paux = pg_aux_env();
+      if (!r.list_v) {
+        dalloc(&r.list_v, (size_t)THIN_CAP);
+        dalloc(&r.list2, (size_t)THIN2_CAP); dalloc(&r.list2_v, (size_t)THIN2_CAP);
+      }
       // persistent grid: every workgroup the CUs hold at once, a multiple of the XCD count
       int occ = 0, occ_ls = 0;
       HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_pgather<false, 0>, PG_WG, 0));
       HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ_ls, k_pgather<true, 0>, PG_WG, 0));
       occ = std::max(1, std::min(occ, occ_ls));
       r.pgrid = ODP_NXCD * std::max(1, C.ncu / ODP_NXCD) * occ;
+      // folded levels need the whole matrix resident, a task per PG_UNIT rows
+      r.fold = s == 1 && !grid_s && src_lo == 0 && src_hi == n && group == ntasks && kw == LEVEL_BLOCK_WORDS &&
+               pg_fold_env();
+      const int T = ntasks;
+      r.cut_full = pg_cut((double)T * r.pupt / ODP_NXCD, 0, r.pgrid / ODP_NXCD);
+      r.cut_fold = pg_cut((double)T * ((T + (T & 1)) / 2) / ODP_NXCD, T & 1 ? 0 : T / 2.0 / ODP_NXCD,
+                          r.pgrid / ODP_NXCD);
     }
     int K = plan.direct;
     while (K >= 2 && (direct_tree(K) > DIRECT_TREE_CAP || !direct_waves(K, kw, group))) K--;
@@ -1003,7 +1086,7 @@ struct Evaluator {
       T.chg1 = T.chg0 + (size_t)segs * n;
       T.act0 = T.chg0 + (size_t)2 * segs * n;
       T.act1 = T.chg0 + (size_t)3 * segs * n;
-      T.asym = r.done + ntasks;
+      T.asym = r.asym;
       T.wgm0 = r.wgm + (size_t)(t % group) * 2 * r.per_task_wg;
       T.wgm1 = T.wgm0 + r.per_task_wg;
       r.l[t] = T.l;
@@ -1063,7 +1146,7 @@ struct Evaluator {
     plan = p;
     if (plan.plan == ODPX_PLAN_LEVEL) setup_level();
     else setup_resident();
-    guess_levels = 0; list_on = true;
+    guess_levels = 0; list_on = true; thin_k = 0;
   }
 
   // ---- evaluation of the adjacency on the device ----
@@ -1121,10 +1204,12 @@ struct Evaluator {
     bool fr = false;                    // frontier-mode level kernel (graphs with many levels)
     int tk = 0;                         // k_tile levels per launch (0: one k_level launch per level)
     int tside = TILE_MIN;               // k_tile's tile side (halo = (64 - side) / 2)
+    bool thin = false;                  // the level before spec runs thin
     int spec = -1;                      // level of the current group launched count-only (expected last)
     bool graphed = false;
     bool pend_fin = false;              // the enqueued batch ends with k_lvfin (sequence number lvseq)
     bool fresh = false, plfresh = false; // the preparation keeps the table / the pair lists
+    bool check = false;                  // ... and checks the table's symmetry
     int first = 0, cnt_t = 0;
     int launched = 0, examined = 0, running = 0, batch_end = 0;
     std::vector<LvTask> sts;
@@ -1171,6 +1256,12 @@ struct Evaluator {
     timed_end(tl);
   }
 
+  // whether the level before a count-only level `spec` lists its unsaturated chunks
+  bool listed_at(int spec) const
+  {
+    return !lv.fr && list_ok() && spec - 1 >= lv.L1 && lr.ntasks < 65536 && n < (1 << 24) && lr.kwp < (1 << 24);
+  }
+
   // gather levels [from, to) of the current group, then the counter and error copies.
   // The count-only level counts just the chunks the level before it listed as
   // unsaturated (plain kernel variant, when that level is a gather level).
@@ -1182,16 +1273,17 @@ struct Evaluator {
       lv_copies(to);
       return;
     }
-    const bool listed = !lv.fr && list_ok() && lv.spec - 1 >= lv.L1 && r.ntasks < 65536 && n < (1 << 24) &&
-                        r.kwp < (1 << 24);
+    const bool listed = listed_at(lv.spec);
     for (int L = from; L < to; L++) {
       int mode = LV_STORE | LV_COUNT;
       if (L == lv.spec) mode = listed ? LV_SPARSE : LV_COUNT;
       else if (listed && L == lv.spec - 1) {
-        mode |= LV_LIST;
-        hipLaunchKernelGGL(k_clear, dim3(LIST_SUBS * LIST_PAD / 256), dim3(256), 0, st, (u64*)nullptr, 0,
-                           (int*)r.list_n, LIST_SUBS * LIST_PAD);
-        HIPC(hipGetLastError());
+        mode = lv.thin ? LV_LIST | LV_THIN : mode | LV_LIST;
+        if (lv.first > 0) {            // the preparation cleared the first group's
+          hipLaunchKernelGGL(k_clear, dim3(LIST_COUNTERS / 256), dim3(256), 0, st, (u64*)nullptr, 0, (int*)r.list_n,
+                             LIST_COUNTERS);
+          HIPC(hipGetLastError());
+        }
       }
       lv_launch(L, mode);
     }
@@ -1229,19 +1321,29 @@ struct Evaluator {
   {
     LevelRun& r = lr;
     const int grid = lv.cnt_t * r.per_task_wg;
-    const LvList lst{r.list, r.list_n, r.list_cap};
+    const bool thin = (mode & LV_THIN) || ((mode & LV_SPARSE) && lv.thin);
+    const u32* asym = pg_on() && r.fold ? r.asym : nullptr;
+    const LvList lst{r.list, r.list_n, thin ? std::min(r.list_cap, THIN_CAP / LIST_SUBS) : r.list_cap,
+                     thin ? r.list_v : nullptr};
+    const LvList lst2{r.list2, r.list_n + LIST_SUBS * LIST_PAD, std::min(r.list_cap, THIN2_CAP / LIST_SUBS), r.list2_v};
     TimedLaunch tl;
     tl.wr = (mode & LV_STORE) ? 1 : 0;
     // k_sparse is timed apart: its work is the listed chunks, not a level
     timed_begin(tl, (mode & LV_SPARSE) ? T_OTHER : T_LEVEL, L, st);
-    if (mode & LV_SPARSE) {
+    if (thin && (mode & LV_SPARSE)) {
+      hipLaunchKernelGGL(k_thin, dim3(std::min(grid, SPARSE_GRID)), dim3(LEVEL_WG), 0, st, r.tasks + lv.first,
+                         lv.cnt_t, L - 1, RING, lst, lst2, asym, (int)((double)n * std::min(r.thin, degree) / std::max(degree, 1)));
+      hipLaunchKernelGGL(k_thin2, dim3(std::min(grid, SPARSE_GRID)), dim3(LEVEL_WG), 0, st, r.tasks + lv.first,
+                         lv.cnt_t, L, RING, lst, lst2, asym);
+    } else if (mode & LV_SPARSE) {
       hipLaunchKernelGGL(k_sparse, dim3(std::min(grid, SPARSE_GRID)), dim3(LEVEL_WG), 0, st,
-                         r.tasks + lv.first, lv.cnt_t, L, RING, lst);
+                         r.tasks + lv.first, lv.cnt_t, L, RING, lst, asym);
     } else if (pg_on()) {
       PgArgs a;
       a.list = r.plist; a.poff = r.ppoff; a.n = n; a.sp = r.psp; a.P = r.parts;
-      a.upt = r.pupt;
-      a.units = (long long)lv.cnt_t * a.upt;
+      a.upt = r.pupt; a.ntasks = lv.cnt_t;
+      a.asym = asym;
+      a.cut_full = r.cut_full; a.cut_fold = r.cut_fold;
       const bool ls = (mode & LV_LIST) != 0;
       auto kern = r.paux == 1 ? (ls ? k_pgather<true, 1> : k_pgather<false, 1>)
                 : r.paux == 16 ? (ls ? k_pgather<true, 16> : k_pgather<false, 16>)
@@ -1263,6 +1365,24 @@ struct Evaluator {
     }
     HIPC(hipGetLastError());
     timed_end(tl);
+  }
+
+  // Neighbours the level before the next evaluation's last one should take: with
+  // a share p of the pairs missing before it, a chunk of 128 is unsaturated after
+  // k neighbours with probability about 128 p^k (what the row itself holds, its
+  // neighbours mostly hold too).  All of them: the level still stores nothing.  Zero when the level leaves too many
+  // pairs for k_thin2's two-step reads.
+  int thin_choice() const
+  {
+    const int L = lv.lmax - 1;
+    if (!lr.parts || L < 1 || L >= LV_MISS_LEVELS || !pg_thin_env()) return 0;
+    const double pairs = (double)n * nsrc, p = lv.miss[L - 1] / pairs;
+    if (p <= 0 || p >= 0.95) return 0;
+    if (lv.miss[L] * dpad * (dpad + 1.0) * (lr.fold ? 0.5 : 1.0) > THIN2_READS) return 0;
+    const int k = std::max(1, (int)std::ceil(std::log(THIN_LEFT / 128) / std::log(p)));
+    // the lists keep their k while the choice stays near it (no rebuild per evaluation)
+    const int kk = lr.thin > 0 && std::abs(k - lr.thin) <= 1 ? lr.thin : k;
+    return std::min(kk, 63);
   }
 
   // the end of a batch that ends at level `to` (the counters of levels
@@ -1305,9 +1425,11 @@ struct Evaluator {
     // the last evaluation ended at level batch_end - 1: expect the same, and
     // launch that level count-only (timed passes keep every level whole)
     lv.spec = spec_at(lv.batch_end) ? lv.batch_end - 1 : -1;
+    lv.thin = listed_at(lv.spec) && pg_on() && thin_k > 0;
     if (lv.first == 0 && lv.graphed) {
       // prepare + the first levels + the first batch + the counter copies as one graph
-      const int be = lv.batch_end, L1 = lv.L1, key = lv_key(be);
+      const int be = lv.batch_end, L1 = lv.L1;
+      const long long key = lv_key(be);
       if (!graph_ready(key))
         capture([&]() { lv_prepare(); lv_level0(); lv_levels(L1, be); }, key);
       else
@@ -1347,27 +1469,27 @@ struct Evaluator {
     return guess_levels > 0 && be == guess_levels && be - 1 >= lv.L1 && !(timed() && !g_stats_live) && !lv.tk;
   }
 
-  // neighbour table, zeroed rings, done and asymmetry flags; in frontier mode the
-  // symmetry check that lets changed rows mark their neighbours (push mode)
+  // neighbour table, zeroed rings and done flags; where the levels use it (folded,
+  // frontier mode) and it is not known, whether the table is symmetric
   void lv_prepare()
   {
     LevelRun& r = lr;
-    prepare(r.cnt, lv.nzero, r.done, r.ntasks + 1, !lv.fresh);
+    prepare(r.cnt, lv.nzero, r.done, r.ntasks + LIST_COUNTERS + (lv.check ? 1 : 0), !lv.fresh);
     if (lv.tk) {
       const int grid = std::min(std::max(1, (n + 255) / 256), 4096);     // a thread per cell
       hipLaunchKernelGGL(k_tgeom, dim3(grid), dim3(256), 0, st, d_nbr, n, dpad, d_row2xy, geo_lmax, d_toff, d_err);
       HIPC(hipGetLastError());
     }
-    if (lv.fr) {
+    if (lv.check) {
       const int64_t total = (int64_t)n * dpad;
       const int grid = (int)std::min<int64_t>(std::max<int64_t>(1, (total + 255) / 256), 4096);
-      hipLaunchKernelGGL(k_symcheck, dim3(grid), dim3(256), 0, st, d_nbr, n, dpad, r.done + r.ntasks);
+      hipLaunchKernelGGL(k_symcheck, dim3(grid), dim3(256), 0, st, d_nbr, n, dpad, r.asym);
       HIPC(hipGetLastError());
     }
     if (pg_on() && !lv.plfresh) {
       // the units' (row, neighbour) pairs grouped by part for k_pgather
       auto kern = dpad + 1 <= 20 ? k_plist<20> : dpad + 1 <= 36 ? k_plist<36> : k_plist<64>;
-      hipLaunchKernelGGL(kern, dim3(r.pupt), dim3(PG_UNIT), 0, st, d_nbr, n, dpad, r.psp, r.parts, r.plist, r.ppoff);
+      hipLaunchKernelGGL(kern, dim3(r.pupt), dim3(PG_UNIT), 0, st, d_nbr, n, dpad, r.psp, r.parts, r.thin, r.plist, r.ppoff);
       HIPC(hipGetLastError());
     }
   }
@@ -1379,12 +1501,12 @@ struct Evaluator {
   // scattered chunks then cost more than a plain count-only level
   bool list_ok() const { return list_on; }
 
-  int lv_key(int be) const
+  long long lv_key(int be) const
   {
-    const int key = 4 * (64 * (16 * (8 * be + (lv.fr ? 1 : 0) + (spec_at(be) ? 2 : 0) + (list_ok() ? 4 : 0)) +
+    const long long key = 8 * (64 * (16 * (8 * be + (lv.fr ? 1 : 0) + (spec_at(be) ? 2 : 0) + (list_ok() ? 4 : 0)) +
                                lv.tk) + lv.tside) +
-                    (lv.fresh ? 1 : 0) + (lv.plfresh ? 2 : 0);
-    return 64 * key + (lv.tk ? std::min(std::max(geo_lmax, 0), 63) : 0);
+                    (lv.fresh ? 1 : 0) + (lv.plfresh ? 2 : 0) + (lv.check ? 4 : 0);
+    return 64 * (64 * key + (lv.tk ? std::min(std::max(geo_lmax, 0), 63) : 0)) + thin_k;
   }
 
   void lv_begin()
@@ -1416,7 +1538,9 @@ struct Evaluator {
     // frontier mode pays off over long level sequences; with few levels every
     // level is dense and the plain kernel is faster
     lv.fr = !lv.tk && (guess_levels == 0 || guess_levels > FRONTIER_MIN_LEVELS);
+    if (thin_k > 0 && thin_k != r.thin) { r.thin = thin_k; pl_fresh = false; }
     lv.plfresh = lv.fresh && pl_fresh;
+    lv.check = (lv.fr || (pg_on() && r.fold)) && !(lv.fresh && asym_fresh);
     lv.graphed = r.group == r.ntasks && use_graph(lv_key(lv.be0));
     if (!lv.graphed) lv_prepare();
     lv.sts.assign(r.ntasks, LvTask{1, 0, 0, 0});
@@ -1430,11 +1554,24 @@ struct Evaluator {
     table_fresh = true;
     table_src = cur_adj();
     if (pg_on()) pl_fresh = true;
+    asym_fresh = lv.check || (lv.fresh && asym_fresh);
   }
 
   bool lv_step()
   {
     LevelRun& r = lr;
+    if (lv.thin && lv.spec >= 0 && r.h_cnt[(size_t)(lv.spec % RING) * r.ntasks + lv.first] == THIN_FAILED) {
+      // more chunks than the lists hold: the thin level again, whole, and the next
+      const int L = lv.spec - 1;
+      for (int k : {L, L + 1}) {
+        hipLaunchKernelGGL(k_clear, dim3((lv.cnt_t + 255) / 256), dim3(256), 0, st,
+                           r.cnt + (size_t)(k % RING) * r.ntasks + lv.first, lv.cnt_t, (int*)nullptr, 0);
+        HIPC(hipGetLastError());
+      }
+      lv.spec = -1; lv.thin = false; thin_k = 0;
+      lv_levels(L, lv.batch_end);
+      return false;
+    }
     for (int t = lv.first; t < lv.first + lv.cnt_t; t++) {
       LvTask& q = lv.sts[t];
       if (!q.running) continue;
@@ -1452,6 +1589,10 @@ struct Evaluator {
     lv.examined = lv.launched;
     if (lv.running > 0 && lv.spec >= 0) {
       // the count-only level was not the last: write its rows now (its counts stand)
+      // (after a thin level, that level's rows first)
+      const bool thin = lv.thin;
+      lv.thin = false;
+      if (thin) lv_launch(lv.spec - 1, LV_STORE);
       lv_launch(lv.spec, LV_STORE);
       lv.spec = -1;
     }
@@ -1469,7 +1610,8 @@ struct Evaluator {
     if (lv.first + r.group >= r.ntasks) {         // the evaluation's last group
       const double frac = lv.lmax >= 1 && lv.lmax - 1 < LV_MISS_LEVELS
                               ? lv.miss[lv.lmax - 1] / ((double)n * (r.kwp / 2) * r.ntasks) : 0;
-      list_on = frac <= (list_on ? 1.0 : 0.5) * list_frac_env();
+      list_on = frac <= (list_on ? 1.0 : 0.5) * list_frac_env(lr.parts ? LIST_MAX_FRAC_PG : LIST_MAX_FRAC);
+      thin_k = thin_choice();
     }
     if (timed()) flush_level_stats(lv.sts.data(), lv.first, lv.cnt_t);
     lv.first += r.group;

@@ -41,6 +41,7 @@ typedef u64 u64v2 __attribute__((ext_vector_type(2)));
 #define LV_COUNT 2          //   ... and add the level's counts (both: a normal level)
 #define LV_LIST 4           //   ... and list the chunks left unsaturated (k_level's LS variant)
 #define LV_SPARSE 8         // the count-only level as k_sparse over that list
+#define LV_THIN 16          // k_pgather: a part of the neighbours, the unsaturated chunks listed with their bits
 
 // chunks (task, row, 16-byte word pair) a level left unsaturated; only those
 // can gain bits at the next level.  The list is LIST_SUBS sub-lists with a
@@ -53,6 +54,7 @@ struct LvList {
   u64* e;              // sub-list s at e + s * cap; entries: task << 48 | row << 24 | word
   u32* n;              // sub-list s's count at n[s * LIST_PAD] (may exceed cap: then no list is used)
   u32 cap;             // entries per sub-list
+  u64x2* v;            // the entries' chunks (16 bytes each), or null
 };
 
 // ---------------------------------------------------------------------------
@@ -60,7 +62,7 @@ struct LvList {
 
 // appends the wave's lanes with `unsat` set to the workgroup's sub-list: one
 // atomic per wave.  Called by whole waves.
-__device__ __forceinline__ void list_append(const LvList& lst, bool unsat, u64 val)
+__device__ __forceinline__ void list_append(const LvList& lst, bool unsat, u64 val, u64 x = 0, u64 y = 0)
 {
   const u64 m = __ballot(unsat);
   if (!m) return;
@@ -70,7 +72,10 @@ __device__ __forceinline__ void list_append(const LvList& lst, bool unsat, u64 v
   b = __builtin_amdgcn_readfirstlane(b);
   if (unsat) {
     const u32 e = b + (u32)__popcll(m & ((1ULL << lane) - 1));
-    if (e < lst.cap) lst.e[(u64)sub * lst.cap + e] = val;
+    if (e < lst.cap) {
+      lst.e[(u64)sub * lst.cap + e] = val;
+      if (lst.v) { u64x2 o; o.x = x; o.y = y; lst.v[(u64)sub * lst.cap + e] = o; }
+    }
   }
 }
 
@@ -229,20 +234,31 @@ __global__ void k_swap(int* adj, int degree, int a, int b, int c, int d, int* er
   }
 }
 
-// Sets *asym when some row u is listed among the neighbours of row r while r
-// is not among u's (entries equal to the row itself are padding).
+// Sets *asym unless the table is symmetric: row u holds row r as many times as
+// row r holds u (entries equal to the row itself are padding).  Counting the
+// repeats makes the property outlive 2-opt swaps: each removes and adds one
+// entry of both directions.  A thread per entry, 16 bytes a load: 41 -> 14 us at
+// n = 65536, d = 16 against a loop over single ids.
 __global__ void k_symcheck(const int* __restrict__ nbr, int n, int dpad, u32* asym)
 {
   const int64_t total = (int64_t)n * dpad;
+  bool bad = false;
   for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
        idx += (int64_t)gridDim.x * blockDim.x) {
-    const int r = (int)(idx / dpad);
+    const int r = (int)((u32)(idx >> 2) / (u32)(dpad >> 2));     // dpad is a multiple of 4; n dpad < 2^33
     const int u = nbr[idx];
     if (u == r) continue;
-    bool found = false;
-    for (int k = 0; k < dpad && !found; k++) found = nbr[(int64_t)u * dpad + k] == r;
-    if (!found) atomicOr(asym, 1u);
+    const int4* own = (const int4*)(nbr + (int64_t)r * dpad);
+    const int4* his = (const int4*)(nbr + (int64_t)u * dpad);
+    int c = 0;
+    for (int k = 0; k < dpad >> 2; k++) {
+      const int4 o = own[k], h = his[k];
+      c += (o.x == u) + (o.y == u) + (o.z == u) + (o.w == u);
+      c -= (h.x == r) + (h.y == r) + (h.z == r) + (h.w == r);
+    }
+    bad = bad || c != 0;
   }
+  if (bad) atomicOr(asym, 1u);
 }
 
 // ---------------------------------------------------------------------------
@@ -557,30 +573,52 @@ __global__ __launch_bounds__(LEVEL_WG) void k_level(const LevelTask* __restrict_
 // (2 MiB at P = 4), which its L2 keeps.  The gathers need no masking (every
 // pair is a 128-byte row read) and none waits for another.  Counts, stop test
 // and listing are k_level's (the plain variant): every result is bit-identical.
+//
+// Folded levels.  With a symmetric table the bit matrix of every level is
+// symmetric: 1024 rows of a 1024-column block are the transpose of the rows
+// and block across the diagonal.  When every block of the matrix is resident
+// (s = 1, 16-word blocks), a level runs the units of one of each such pair and
+// stores both: a unit's rows and, transposed in LDS, its mirror's.  Its bits count
+// for both blocks.  Half the gathers for 6 us of mirroring a unit of 50:
+// a level of n = 65536, d = 16 went from 677 to 459 us.  Of a block t the rows
+// of blocks t, t + 1, ..., t + (T - 1) / 2 (mod T, T blocks) run, so every block has
+// as many and an XCD still works on one block's slab at a time; for even T the
+// rows t + T / 2 of the first half of the blocks come last.  Whether the table is
+// symmetric is read on the device (k_symcheck); other tables run every unit.
 
 #define PG_MAXP 4
+#define PG_SUB 8             // pieces of a unit's rows in its offsets (128 rows each)
+#define PG_OFF (2 * PG_MAXP * PG_SUB + 1)   // offsets of a unit's pair list: per part, its thin pairs and the
+                             // others, per piece; then its end
 #ifndef PG_SLOTS
 #define PG_SLOTS 12          // gathers a wave keeps in flight (registers: 4 per slot)
 #endif
 #define PG_CH (8 * PG_SLOTS) // pairs of a chunk
 #define PG_NL ((PG_CH + 63) / 64)
-#define PG_UNIT 1024         // rows of a unit, 128 KiB of LDS rows: one workgroup per CU
-#ifndef PG_WG
-#define PG_WG 1024           // threads of the workgroup (a divisor of PG_UNIT)
-#endif
+#define PG_UNIT 1024         // rows of a unit (and sources of a 16-word block, which a folded unit mirrors to):
+                             // 128 KiB of LDS rows, one workgroup per CU.  With 512 rows and two workgroups, whose
+                             // phases drift apart, the XCD's L2 holds more than one part: 762 against 665 us a level
+#define PG_WG PG_UNIT        // threads of the workgroup: 64 rows a wave at the end
+#define PG_CUT_MAX 3         // log2 of the pieces of a unit: two waves' rows are the smallest
 
 struct PgArgs {
   const u32* list;       // per unit, parts in order: (row in unit) << 22 | neighbour
-  const int* poff;       // per unit: P + 1 offsets into its list (relative to unit * PG_UNIT * sp)
+  const int* poff;       // per unit PG_OFF offsets into its list (relative to unit * PG_UNIT * sp): piece k of
+                         // part p's thin pairs starts at [2 p * PG_SUB + k], of its others at [(2 p + 1) * PG_SUB + k],
+                         // the list ends at [2 P * PG_SUB]
   int n, sp, P;
   int upt;               // units per task: ceil(n / PG_UNIT)
-  long long units;       // tasks x upt
+  int ntasks;
+  const u32* asym;       // folded levels unless *asym (null: never; needs one task per PG_UNIT rows)
+  int cut_full, cut_fold;  // log2 of the pieces a unit of the last, partly filled round is cut into (<= PG_CUT_MAX)
 };
 
 // One workgroup of PG_UNIT threads per unit, a thread per row: the row's
 // distinct neighbours and the row itself (padding entries are the row), their
 // parts, a scan of the rows' run lengths per part, and the unit's pairs
-// grouped by part (in any order within a part) with the part offsets.
+// grouped by part with the part offsets.  A part's thin pairs come first: the
+// row itself and its first `thin` neighbours, in the order of the parts (a thin
+// level, LV_THIN, takes those alone); rows ascend within either group.
 // DMAX >= dpad + 1 bounds the ids a row holds in registers.
 //
 // A device swap (or a small change of an uploaded table) hands the changed
@@ -592,9 +630,10 @@ struct PlMove { int row[PL_MOVE_MAX], pos[PL_MOVE_MAX], from[PL_MOVE_MAX], to[PL
 // one unit's pair lists (a workgroup of PG_UNIT threads, unit u)
 template <int DMAX>
 __device__ __forceinline__ void plist_unit(const int* __restrict__ nbr, int n, int dpad, int sp, int P,
-                                           u32* __restrict__ list, int* __restrict__ poff, int u, const PlMove& mv)
+                                           int thin, u32* __restrict__ list, int* __restrict__ poff, int u,
+                                           const PlMove& mv)
 {
-  __shared__ u64 wtot[PG_UNIT / 64];
+  __shared__ u64 wtot[2][PG_UNIT / 64];
   const int t = threadIdx.x, r = u * PG_UNIT + t, lane = t & 63, wave = t >> 6;
   // the row's table entries, 16 bytes a load (dpad is a multiple of 4), every
   // thread loading (a row past n reads the last row's): a load under a lane
@@ -635,43 +674,73 @@ __device__ __forceinline__ void plist_unit(const int* __restrict__ nbr, int n, i
     for (int k = 0; k < j; k++) dup = dup || id[k] == id[j];
     if (dup) id[j] = -1;
   }
-  u64 run = 0;                                      // four 16-bit counts (a unit holds < 65536 pairs of a part)
+  // per part, how many of the row's ids are thin: its own (once), and the first
+  // `thin` neighbours in the order of the parts
+  u64 all = 0, own = 0;                             // four 16-bit counts each (a unit holds < 65536 pairs of a part)
 #pragma unroll
   for (int j = 0; j < DMAX; j++)
-    if (id[j] >= 0) run += 1ULL << (16 * part(id[j]));
-  // inclusive scan over the unit's rows: within the wave, then the waves before
-  u64 inc = run;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const u64 v = __shfl_up(inc, o, 64);
-    if (lane >= o) inc += v;
-  }
-  if (lane == 63) wtot[wave] = inc;
-  __syncthreads();
-  u64 tot = 0;
-  for (int i = 0; i < PG_UNIT / 64; i++) {
-    const u64 v = wtot[i];
-    if (i < wave) inc += v;
-    tot += v;
-  }
-  __syncthreads();                                  // wtot is free for the next unit
-  u32* ul = list + (int64_t)u * PG_UNIT * sp;
-  int pos[PG_MAXP], base = 0;
+    if (id[j] >= 0) {
+      const u64 one = 1ULL << (16 * part(id[j]));
+      if (id[j] == r) own += one; else all += one;
+    }
+  u64 run[2] = {own, all};
+  int left = thin;
 #pragma unroll
   for (int p = 0; p < PG_MAXP; p++) {
-    pos[p] = base + (int)((inc >> (16 * p)) & 0xffff) - (int)((run >> (16 * p)) & 0xffff);
-    if (t == 0 && p < P) poff[u * (PG_MAXP + 1) + p] = base;
-    base += p < P ? (int)((tot >> (16 * p)) & 0xffff) : 0;
+    const int k = min((int)((all >> (16 * p)) & 0xffff), left);
+    left -= k;
+    run[0] += (u64)k << (16 * p);
+    run[1] -= (u64)k << (16 * p);
   }
-  if (t == 0) poff[u * (PG_MAXP + 1) + P] = base;
+  const u64 quota = run[0] - own;
+  // inclusive scans over the unit's rows: within the wave, then the waves before
+  u64 inc[2] = {run[0], run[1]}, tot[2] = {0, 0};
+#pragma unroll
+  for (int c = 0; c < 2; c++) {
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const u64 v = __shfl_up(inc[c], o, 64);
+      if (lane >= o) inc[c] += v;
+    }
+    if (lane == 63) wtot[c][wave] = inc[c];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < 2; c++)
+    for (int i = 0; i < PG_UNIT / 64; i++) {
+      const u64 v = wtot[c][i];
+      if (i < wave) inc[c] += v;
+      tot[c] += v;
+    }
+  __syncthreads();                                  // wtot is free for the next unit
+  u32* ul = list + (int64_t)u * PG_UNIT * sp;
+  int pos[PG_MAXP][2], base = 0;
+#pragma unroll
+  for (int p = 0; p < PG_MAXP; p++)
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      pos[p][c] = base + (int)((inc[c] >> (16 * p)) & 0xffff) - (int)((run[c] >> (16 * p)) & 0xffff);
+      if (t % (PG_UNIT / PG_SUB) == 0 && p < P)
+        poff[u * PG_OFF + (2 * p + c) * PG_SUB + t / (PG_UNIT / PG_SUB)] = pos[p][c];
+      base += p < P ? (int)((tot[c] >> (16 * p)) & 0xffff) : 0;
+    }
+  if (t == 0) poff[u * PG_OFF + 2 * P * PG_SUB] = base;
+  int need[PG_MAXP];                                // thin neighbours still to place
+#pragma unroll
+  for (int p = 0; p < PG_MAXP; p++) need[p] = (int)((quota >> (16 * p)) & 0xffff);
 #pragma unroll
   for (int j = 0; j < DMAX; j++)
     if (id[j] >= 0) {
       const int q = part(id[j]);
+      const bool mine = id[j] == r;
       int at = 0;
 #pragma unroll
       for (int p = 0; p < PG_MAXP; p++)
-        if (p == q) at = pos[p]++;
+        if (p == q) {
+          const bool th = mine || need[p] > 0;
+          at = th ? pos[p][0]++ : pos[p][1]++;
+          need[p] -= th && !mine ? 1 : 0;
+        }
       ul[at] = ((u32)t << 22) | (u32)id[j];
     }
 }
@@ -679,11 +748,11 @@ __device__ __forceinline__ void plist_unit(const int* __restrict__ nbr, int n, i
 // every unit (workgroup u builds unit u)
 template <int DMAX>
 __global__ __launch_bounds__(PG_UNIT) void k_plist(const int* __restrict__ nbr, int n, int dpad, int sp, int P,
-                                                   u32* __restrict__ list, int* __restrict__ poff)
+                                                   int thin, u32* __restrict__ list, int* __restrict__ poff)
 {
   PlMove none;
   none.cnt = 0;
-  plist_unit<DMAX>(nbr, n, dpad, sp, P, list, poff, blockIdx.x, none);
+  plist_unit<DMAX>(nbr, n, dpad, sp, P, thin, list, poff, blockIdx.x, none);
 }
 
 // Entries at positions the host found (a 2-opt move, checked with k_swap's
@@ -693,7 +762,7 @@ __global__ __launch_bounds__(PG_UNIT) void k_plist(const int* __restrict__ nbr, 
 // applying the entries to its rows as it reads them.  With mv.cnt = 0 it only
 // rebuilds the units.
 struct PlUnits { int u[PL_MOVE_MAX]; int cnt; };
-struct PlArgs { const int* nbr; int n, dpad, sp, P; u32* list; int* poff; };
+struct PlArgs { const int* nbr; int n, dpad, sp, P, thin; u32* list; int* poff; };
 
 template <int DMAX>
 __global__ __launch_bounds__(PG_UNIT) void k_swap_at(int* adj, int degree, SwapTables tb, PlMove mv, PlUnits units,
@@ -707,16 +776,90 @@ __global__ __launch_bounds__(PG_UNIT) void k_swap_at(int* adj, int degree, SwapT
     if (tb.t32 && tb.t32[k] == mv.from[e]) tb.t32[k] = mv.to[e];
   }
   if ((int)blockIdx.x < units.cnt)
-    plist_unit<DMAX>(pl.nbr, pl.n, pl.dpad, pl.sp, pl.P, pl.list, pl.poff, units.u[blockIdx.x], mv);
+    plist_unit<DMAX>(pl.nbr, pl.n, pl.dpad, pl.sp, pl.P, pl.thin, pl.list, pl.poff, units.u[blockIdx.x], mv);
 }
 
 typedef u32 u32x4v __attribute__((ext_vector_type(4)));
 typedef u32 u32x2v __attribute__((ext_vector_type(2)));
 
+// Bits (i, j) of a 64 x 64 bit block swapped, for the block's word w and w + 1:
+// before, x[g] of lane l holds row 8 g + l / 8 of the word pair l % 8; after, it
+// holds column 8 g + l / 8 of the pair's words as 64 bits of rows.  Six
+// exchanges of an index bit with a bit position: row bits 5, 4 and 3 lie in g
+// (registers: a renaming and byte permutes), bits 2, 1 and 0 in lane bits 5, 4
+// and 3.
+__device__ __forceinline__ void swap_bits(u32& p, u32& q, u32 m, int sh)   // q's bits under m with p's sh above
+{
+  const u32 a = (p & m) | ((q & m) << sh), b = ((p >> sh) & m) | (q & ~m);
+  p = a; q = b;
+}
+__device__ __forceinline__ void transpose64(u32 (&lo)[8], u32 (&hi)[8], int lane)
+{
+#pragma unroll
+  for (int g = 0; g < 4; g++) { const u32 t = hi[g]; hi[g] = lo[g + 4]; lo[g + 4] = t; }
+  auto perm2 = [](u32& p, u32& q, u32 s0, u32 s1) {
+    const u32 a = __builtin_amdgcn_perm(q, p, s0), b = __builtin_amdgcn_perm(q, p, s1);
+    p = a; q = b;
+  };
+#pragma unroll
+  for (int g = 0; g < 8; g++)
+    if (!(g & 2)) {
+      perm2(lo[g], lo[g + 2], 0x05040100u, 0x07060302u);
+      perm2(hi[g], hi[g + 2], 0x05040100u, 0x07060302u);
+    }
+#pragma unroll
+  for (int g = 0; g < 8; g += 2) {
+    perm2(lo[g], lo[g + 1], 0x06020400u, 0x07030501u);
+    perm2(hi[g], hi[g + 1], 0x06020400u, 0x07030501u);
+  }
+  // a pair of registers: the swap brings both rows of an exchange into one
+  // lane, and back
+  auto lanes32 = [](u32& p, u32& q) {
+    auto r = __builtin_amdgcn_permlane32_swap(p, q, false, false);
+    p = r[0]; q = r[1];
+  };
+  auto lanes16 = [](u32& p, u32& q) {
+    auto r = __builtin_amdgcn_permlane16_swap(p, q, false, false);
+    p = r[0]; q = r[1];
+  };
+#pragma unroll
+  for (int g = 0; g < 8; g++) {
+    lanes32(lo[g], hi[g]); swap_bits(lo[g], hi[g], 0x0f0f0f0fu, 4); lanes32(lo[g], hi[g]);
+    lanes16(lo[g], hi[g]); swap_bits(lo[g], hi[g], 0x33333333u, 2); lanes16(lo[g], hi[g]);
+  }
+  const bool odd = (lane & 8) != 0;
+  const u32 keep = odd ? 0xaaaaaaaau : 0x55555555u, rot = odd ? 1u : 31u;
+  auto lanes8 = [&](u32& p) {                          // lane ^ 8: a rotation by 8 within 16 lanes
+    const u32 y = (u32)__builtin_amdgcn_update_dpp(0, (int)p, 0x128, 0xf, 0xf, false);
+    p = (p & keep) | (__builtin_amdgcn_alignbit(y, y, rot) & ~keep);
+  };
+#pragma unroll
+  for (int g = 0; g < 8; g++) { lanes8(lo[g]); lanes8(hi[g]); }
+}
+
+// the stop test of k_level at this level
+__device__ __forceinline__ bool task_stops(const LevelTask& T, int level, int ring)
+{
+  const u64 c1 = T.cnt[(int64_t)((level - 1) % ring) * T.cstride];
+  return c1 == (u64)T.n * (u64)T.l || (level >= 2 && c1 == T.cnt[(int64_t)((level - 2) % ring) * T.cstride]);
+}
+
+// A workgroup barrier that orders LDS alone: __syncthreads also waits for the
+// global stores, and k_pgather's rows, which nothing in the launch reads, may
+// drain while the next unit gathers.
+__device__ __forceinline__ void lds_barrier()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 // Persistent: workgroup b runs on XCD b % 8 and takes every (gridDim.x / 8)-th
 // unit of its XCD's contiguous range of units (a unit: PG_UNIT rows of one
 // task), so the XCD's workgroups sweep that range together; any grid that is a
-// multiple of 8 works.  The gathers are buffer loads with cache policy AUX
+// multiple of 8 works.  The units of the last round, when they do not fill it,
+// are cut into pieces of their rows (2^cut of them) dealt over the workgroups.
+// The gathers are buffer loads with cache policy AUX
 // (0: default; 1: sc0, 16: sc1, 2: nt), bounded by the slab (out-of-range
 // offsets read zero).
 template <bool LS, int AUX>
@@ -725,54 +868,99 @@ __global__ __launch_bounds__(PG_WG) void k_pgather(const LevelTask* __restrict__
 {
   __shared__ u64x2 acc[PG_UNIT * 8];                  // row r of the unit at [8 r, 8 r + 8)
   __shared__ u64 s_pop[PG_WG / 64];
+  __shared__ int s_off[PG_OFF], s_next;
+  __shared__ int2 s_chunk[PG_UNIT * 64 / PG_CH + 2 * PG_MAXP];   // chunks of a unit (at most 64 pairs a row, rounded up per group)
   const int x = blockIdx.x % ODP_NXCD, wi = blockIdx.x / ODP_NXCD, nwx = gridDim.x / ODP_NXCD;
-  const long long u_lo = a.units * x / ODP_NXCD, u_hi = a.units * (x + 1) / ODP_NXCD;
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane_ = tid & 63, lane = lane_;
   const int nw = PG_WG / 64;
+  static_assert(PG_UNIT / (PG_WG / 64) == 64, "a wave stores and transposes 64 rows of a unit");
   const bool count = (mode & LV_COUNT) != 0, store = (mode & LV_STORE) != 0;
   const int w = 2 * (lane & 7);                       // the lane's two words of a row
-  for (long long u = u_lo + wi; u < u_hi; u += nwx) { // uniform
-    const int t = (int)(u / a.upt), ur = (int)(u - (long long)t * a.upt);
-    const LevelTask& T = tasks[t];
-    if (*T.done) continue;
-    const u64 c1 = T.cnt[(int64_t)((level - 1) % ring) * T.cstride];
-    if (c1 == (u64)T.n * (u64)T.l || (level >= 2 && c1 == T.cnt[(int64_t)((level - 2) % ring) * T.cstride])) {
-      if (tid == 0) *T.done = 1;
-      continue;
+  const bool fold = a.asym && __builtin_amdgcn_readfirstlane(*a.asym) == 0;
+  if (fold) {
+    // a unit stands for two blocks, so all run until none has to
+    bool run = false;
+    for (int t = lane; t < a.ntasks; t += 64) {
+      const LevelTask& T = tasks[t];
+      const bool stop = *T.done || task_stops(T, level, ring);
+      run = run || !stop;
+      if (blockIdx.x == 0 && wave == 0) {
+        if (stop) *T.done = 1;
+        if (count) T.cnt[(int64_t)((level + 1) % ring) * T.cstride] = 0;
+      }
     }
-    if (count && ur == 0 && tid == 0) T.cnt[(int64_t)((level + 1) % ring) * T.cstride] = 0;
+    if (!__any(run)) return;                          // the same in every wave of the launch
+  }
+  const int T2 = a.ntasks, hs = (T2 + (T2 & 1)) / 2;  // folded: blocks of rows a block runs in the rounds
+  const int main_n = fold ? T2 * hs : a.ntasks * a.upt, extra_n = fold && !(T2 & 1) ? T2 / 2 : 0;
+  const int u_lo = (int)((int64_t)main_n * x / ODP_NXCD), u_hi = (int)((int64_t)main_n * (x + 1) / ODP_NXCD);
+  const int e_lo = extra_n * x / ODP_NXCD, e_hi = extra_n * (x + 1) / ODP_NXCD;
+  const int rounds = (u_hi - u_lo) / nwx, rest = (u_hi - u_lo) - rounds * nwx;
+  const int cut = fold ? a.cut_fold : a.cut_full, pieces = (rest + e_hi - e_lo) << cut;
+  for (int it = 0;; it++) {                           // uniform
+    int u, s0 = 0, s1 = PG_SUB;                       // the unit and its piece [s0, s1) in PG_SUB-ths
+    if (it < rounds) {
+      u = u_lo + it * nwx + wi;
+    } else {
+      const int p = (it - rounds) * nwx + wi, k = p >> cut;
+      if (p >= pieces) break;
+      u = k < rest ? u_lo + rounds * nwx + k : main_n + e_lo + (k - rest);
+      s0 = (p & ((1 << cut) - 1)) * (PG_SUB >> cut);
+      s1 = s0 + (PG_SUB >> cut);
+    }
+    int t, ur;
+    if (!fold) { t = u / a.upt; ur = u - t * a.upt; }
+    else if (u < main_n) { t = u / hs; ur = t + (u - t * hs); if (ur >= T2) ur -= T2; }
+    else { t = u - main_n; ur = t + T2 / 2; }
+    const LevelTask& T = tasks[t];
+    if (!fold) {
+      if (*T.done) continue;
+      if (task_stops(T, level, ring)) {
+        if (tid == 0) *T.done = 1;
+        continue;
+      }
+      if (count && ur == 0 && tid == 0) T.cnt[(int64_t)((level + 1) % ring) * T.cstride] = 0;
+    }
+    const bool mirror = fold && ur != t;
     const u64* __restrict__ cur = (level & 1) ? T.buf1 : T.buf0;
     u64* __restrict__ nxt = (level & 1) ? T.buf0 : T.buf1;
     const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc((void*)cur, 0, a.n * 128, 0x00020000);
     const u64 f0 = full_word(T.l, w), f1 = full_word(T.l, w + 1);
-#pragma unroll
-    for (int i = tid; i < PG_UNIT * 8; i += PG_WG) { acc[i].x = 0; acc[i].y = 0; }
-    __syncthreads();
+    for (int i = s0 * 128 * 8 + tid; i < s1 * 128 * 8; i += PG_WG) { acc[i].x = 0; acc[i].y = 0; }
     const u32* __restrict__ ul = a.list + (int64_t)ur * PG_UNIT * a.sp;
-    const int* po = a.poff + ur * (PG_MAXP + 1);
-    // the parts in order; within a part the waves take chunks of PG_CH pairs in
-    // turn.  A chunk's PG_SLOTS gathers (eight rows each) are in flight while
-    // the wave ORs in the previous chunk's rows: a slot's next gather is issued
+    const int* po = a.poff + ur * PG_OFF;
+    // the parts in order; the waves take the chunks of PG_CH pairs of all parts
+    // from a counter, two chunks ahead (dealt in turn, wave 0, which the SIMD
+    // prefers, waited 11 us of a unit's 57 for the others at the barrier: a folded
+    // level 478 -> 459 us).  A chunk's PG_SLOTS gathers (eight rows each) are in
+    // flight while the wave ORs in the previous chunk's rows: a slot's next gather is issued
     // as soon as its rows are ORed in, and a chunk's pairs are loaded a chunk
     // ahead.  (Waiting slot by slot instead of once per chunk was measured
     // slower.)  The in-flight rows live in registers: PG_SLOTS sets how many.
     const u32 SENT = 0xffffffffu;
-    // the unit's part offsets, read once (no memory read in the chunk loop may
-    // make the wave wait for the gathers in flight)
-    const int b0 = __builtin_amdgcn_readfirstlane(po[0]), b1 = __builtin_amdgcn_readfirstlane(po[1]);
-    const int b2 = a.P > 1 ? __builtin_amdgcn_readfirstlane(po[2]) : b1;
-    const int b3 = a.P > 2 ? __builtin_amdgcn_readfirstlane(po[3]) : b2;
-    const int b4 = a.P > 3 ? __builtin_amdgcn_readfirstlane(po[4]) : b3;
-    // The XCD's workgroups take its units in rounds; every other round sweeps
-    // the parts backwards, so it starts with the part the round before ended
-    // with, whose rows are still in L2.
-    const bool rev = (((u - u_lo - wi) / nwx) & 1) != 0;
-    auto boff = [&](int p) { return p == 0 ? b0 : p == 1 ? b1 : p == 2 ? b2 : p == 3 ? b3 : b4; };
-    auto pbeg = [&](int pp) { return boff(rev ? a.P - 1 - pp : pp); };
-    auto pend = [&](int pp) { return boff(rev ? a.P - pp : pp + 1); };
-    auto advance = [&](int& pp, int& cc) {                 // uniform
-      while (pp < a.P && cc >= pend(pp)) { pp++; if (pp < a.P) cc = pbeg(pp) + wave * PG_CH; }
-    };
+    // The chunks of the piece, part after part, listed in LDS (a chunk's pairs
+    // [first, end)); no table read from memory in the chunk loop, which would
+    // make the wave wait for the gathers in flight.  The XCD's workgroups take
+    // its units in rounds; every other round sweeps the parts backwards, so it
+    // starts with the part the round before ended with, whose rows are still in
+    // L2.
+    if (tid < PG_OFF) s_off[tid] = po[tid];               // (entries past 2 P * PG_SUB are not used)
+    if (tid == 0) s_next = 3 * nw;
+    lds_barrier();
+    int nch = 0;
+    for (int pp = 0; pp < 2 * a.P; pp++) {                // uniform
+      const int p = it & 1 ? 2 * a.P - 1 - pp : pp;
+      if ((p & 1) && (mode & LV_THIN)) continue;
+      const int lo = __builtin_amdgcn_readfirstlane(s_off[p * PG_SUB + s0]);
+      const int hi = __builtin_amdgcn_readfirstlane(s_off[p * PG_SUB + s1]);
+      const int nc = (int)((u32)(hi - lo + PG_CH - 1) / PG_CH);
+      for (int k = tid; k < nc; k += PG_WG) {
+        s_chunk[nch + k].x = lo + k * PG_CH;
+        s_chunk[nch + k].y = min(lo + (k + 1) * PG_CH, hi);
+      }
+      nch += nc;
+    }
+    lds_barrier();                                      // acc is clear, the chunks are listed
     // a chunk's pairs, 64 per register (every lane loads: an idle one the unit's
     // first entry).  Lane group g (eight lanes, one row) takes the chunk's pairs
     // [g PG_SLOTS, (g + 1) PG_SLOTS), one per slot: a row's pairs of a part are
@@ -780,13 +968,16 @@ __global__ __launch_bounds__(PG_WG) void k_pgather(const LevelTask* __restrict__
     // different rows and their ORs no two lanes' same LDS word.  Register h,
     // lane l holds the pair of slot 8 h + l / 8, group l % 8.
     struct Pairs { u32 v[PG_NL]; };
-    auto pairs = [&](int pp, int cc) -> Pairs {
+    auto pairs = [&](int k) -> Pairs {
       Pairs r;
+      // past the last chunk (a piece may have none, and s_chunk[0] is then unwritten): no pair
+      const int2 c = s_chunk[k < nch ? k : 0];
+      const int cc = k < nch ? c.x : 0, ce = k < nch ? c.y : 0;
 #pragma unroll
       for (int h = 0; h < PG_NL; h++) {
         const int q = 8 * h + (lane >> 3);
         const int i = cc + (lane & 7) * PG_SLOTS + q;
-        const bool ok = pp < a.P && q < PG_SLOTS && i < pend(pp);
+        const bool ok = q < PG_SLOTS && i < ce;
         const u32 v = ul[ok ? i : 0];
         r.v[h] = ok ? v : SENT;
       }
@@ -803,18 +994,15 @@ __global__ __launch_bounds__(PG_WG) void k_pgather(const LevelTask* __restrict__
       const u32x4v v = __builtin_amdgcn_raw_buffer_load_b128(src, (int)off, 0, AUX);
       gv[q].x = ((u64)v.y << 32) | v.x; gv[q].y = ((u64)v.w << 32) | v.z;
     };
-    int p0 = 0, k0 = pbeg(0) + wave * PG_CH;
-    advance(p0, k0);
-    int p1 = p0, k1 = k0 + nw * PG_CH;
-    advance(p1, k1);
-    const Pairs first = pairs(p0, k0);
-    Pairs next = pairs(p1, k1);
+    const Pairs first = pairs(wave);
+    Pairs next = pairs(wave + nw);
 #pragma unroll
     for (int q = 0; q < PG_SLOTS; q++) issue(first, q);
-    while (p0 < a.P) {                                    // wave-uniform: this chunk's gathers are in flight
-      int p2 = p1, k2 = k1 + nw * PG_CH;
-      advance(p2, k2);
-      const Pairs after = pairs(p2, k2);
+    int k0 = wave, k1 = wave + nw, k2 = wave + 2 * nw;    // this chunk, the next (its pairs loaded) and the one after
+    while (k0 < nch) {                                    // wave-uniform: this chunk's gathers are in flight
+      const Pairs after = pairs(k2);
+      int k3 = 0;
+      if (lane == 0) k3 = atomicAdd(&s_next, 1);
       // Rows are 128 bytes apart: a row's eight lanes meet 16 of the 64 banks
       // with the first word of their pieces, the other 16 of the row's half of
       // the banks with the second.  A row with bit 1 set ORs its second word
@@ -831,33 +1019,80 @@ __global__ __launch_bounds__(PG_WG) void k_pgather(const LevelTask* __restrict__
         }
         issue(next, q);                                     // all SENT past the last chunk
       }
-      p0 = p1; k0 = k1; p1 = p2; k1 = k2; next = after;
+      next = after;
+      k0 = k1; k1 = k2; k2 = __builtin_amdgcn_readfirstlane(k3);
     }
-    __syncthreads();
-    // the unit's rows: written, counted, listed; wave w takes rows [R w, R w + R), R = PG_UNIT / nw
+    lds_barrier();
+    // the unit's rows: written, counted, listed; wave w takes rows [64 w, 64 w + 64)
     u64 pop = 0;
-    for (int g = 0; g < PG_UNIT / nw / 8; g++) {
-      const int lr = wave * (PG_UNIT / nw) + g * 8 + (lane >> 3), r = ur * PG_UNIT + lr;
-      const bool valid = r < a.n;
-      const u64x2 v = acc[lr * 8 + (w >> 1)];
-      if (valid) {
-        if (store) {
-          u64v2 o; o.x = v.x; o.y = v.y;
-          __builtin_nontemporal_store(o, (u64v2*)(nxt + (int64_t)r * 16 + w));   // streamed past L2
+    // the lane's addresses of this part are computed here: hoisted out of the
+    // unit loop they would take the registers of the gathers in flight
+    int lane = lane_;
+    asm volatile("" : "+v"(lane));
+    const int w = 2 * (lane & 7);
+    const bool mine = (wave >> 1) >= s0 && (wave >> 1) < s1;   // two waves' rows are a piece
+    u32 lo0[8], hi0[8], lo1[8], hi1[8];
+    if (mine) {
+#pragma unroll
+      for (int g = 0; g < 8; g++) {
+        const int lr = wave * 64 + g * 8 + (lane >> 3), r = ur * PG_UNIT + lr;
+        const bool valid = r < a.n;
+        const u64x2 v = acc[lr * 8 + (w >> 1)];
+        lo0[g] = (u32)v.x; hi0[g] = (u32)(v.x >> 32); lo1[g] = (u32)v.y; hi1[g] = (u32)(v.y >> 32);
+        if (valid) {
+          if (store) {
+            u64v2 o; o.x = v.x; o.y = v.y;
+            __builtin_nontemporal_store(o, (u64v2*)(nxt + (int64_t)r * 16 + w));   // streamed past L2
+          }
+          pop += (u64)(__popcll(v.x) + __popcll(v.y));
         }
-        pop += (u64)(__popcll(v.x) + __popcll(v.y));
+        if (LS) list_append(lst, valid && !(v.x == f0 && v.y == f1), ((u64)t << 48) | ((u64)r << 24) | (u64)w, v.x, v.y);
       }
-      if (LS) list_append(lst, valid && !(v.x == f0 && v.y == f1), ((u64)t << 48) | ((u64)r << 24) | (u64)w);
     }
     if (count) {
       pop = wave_sum(pop);
       if (lane == 0) s_pop[wave] = pop;
     }
-    __syncthreads();                                  // acc and s_pop are free for the next unit
+    lds_barrier();                                  // acc is read, s_pop written
     if (count && tid == 0) {
       u64 sum = 0;
       for (int i = 0; i < nw; i++) sum += s_pop[i];
-      if (sum) atomicAdd(&T.cnt[(int64_t)(level % ring) * T.cstride], sum);
+      if (sum) {
+        atomicAdd(&T.cnt[(int64_t)(level % ring) * T.cstride], sum);
+        if (mirror) atomicAdd(&tasks[ur].cnt[(int64_t)(level % ring) * T.cstride], sum);
+      }
+    }
+    if (mirror && store) {                            // uniform
+      // The mirror's row c (column c of this unit) holds wave j's 64 rows as its
+      // word j, at position j ^ swz(c) of the row in LDS: the 64 lanes of a store
+      // have one j and rows that differ in bits 0-2 and 7-9, and bit 0 and swz
+      // spread them over all banks.
+      auto swz = [](int c) { return ((c >> 1) & 3) | (((c >> 7) & 3) << 2); };
+      if (mine) {
+        transpose64(lo0, hi0, lane);
+        transpose64(lo1, hi1, lane);
+        u64* words = (u64*)acc;
+#pragma unroll
+        for (int g = 0; g < 8; g++) {
+          const int c = 64 * w + 8 * g + (lane >> 3);
+          words[c * 16 + (wave ^ swz(c))] = ((u64)hi0[g] << 32) | lo0[g];
+          words[(c + 64) * 16 + (wave ^ swz(c + 64))] = ((u64)hi1[g] << 32) | lo1[g];
+        }
+      }
+      lds_barrier();
+      u64* __restrict__ mnxt = (level & 1) ? tasks[ur].buf0 : tasks[ur].buf1;
+      const int kq = lane & 7;                        // the lane's word pair of a row: waves 2 kq, 2 kq + 1
+      if (kq >= s0 && kq < s1) {
+#pragma unroll
+        for (int g = 0; g < 8; g++) {
+          const int c = wave * 64 + g * 8 + (lane >> 3), r = t * PG_UNIT + c, f = swz(c);
+          const u64x2 v = acc[c * 8 + (kq ^ (f >> 1))];
+          u64v2 o;
+          o.x = f & 1 ? v.y : v.x; o.y = f & 1 ? v.x : v.y;
+          if (r < a.n) __builtin_nontemporal_store(o, (u64v2*)(mnxt + (int64_t)r * 16 + w));
+        }
+      }
+      lds_barrier();                                // acc is free for the next unit
     }
   }
 }
@@ -968,7 +1203,7 @@ __device__ __forceinline__ int chunk_gain(const LevelTask& T, int level, int r, 
   return __popcll(x.x) + __popcll(x.y) - __popcll(x0.x) - __popcll(x0.y);
 }
 
-// adds each lane's gain to its task's count of the level: one wave sum and one
+// adds each lane's gain (or, negative, loss) to its task's count of the level: one wave sum and one
 // atomic per task among the lanes with a gain (listed chunks next to each
 // other in the list can come from several tasks; an atomic per lane on the
 // few task counters had serialised, 15 ms for 3 M chunks at n = 20000).
@@ -980,22 +1215,51 @@ __device__ __forceinline__ void add_gains(const LevelTask* __restrict__ tasks, i
   for (u64 m = __ballot(left); m; m = __ballot(left)) {   // wave-uniform
     const int t0 = __shfl(t, __ffsll((long long)m) - 1, 64);
     const bool mine = left && t == t0;
-    const u64 s = wave_sum(mine ? (u64)gain : 0ULL);
+    const u64 s = wave_sum(mine ? (u64)(long long)gain : 0ULL);
     if ((threadIdx.x & 63) == 0) atomicAdd(&tasks[t0].cnt[(int64_t)(level % ring) * tasks[t0].cstride], s);
     left = left && !mine;
   }
 }
 
-// the stop test of k_level at this level
-__device__ __forceinline__ bool task_stops(const LevelTask& T, int level, int ring)
-{
-  const u64 c1 = T.cnt[(int64_t)((level - 1) % ring) * T.cstride];
-  return c1 == (u64)T.n * (u64)T.l || (level >= 2 && c1 == T.cnt[(int64_t)((level - 2) % ring) * T.cstride]);
-}
+// A list's sub-lists read as one: lane s holds sub-list s's count (LIST_SUBS is
+// the wave size) and the count of the sub-lists before it; entry e is in the
+// last sub-list that starts at or below e.
+struct ListView {
+  u32 excl, total, cap;
+  bool over;                                          // a sub-list passed its capacity
+  __device__ __forceinline__ ListView(const LvList& lst, int lane)
+  {
+    static_assert(LIST_SUBS == 64, "one sub-list per lane");
+    const u32 cnt = lst.n[lane * LIST_PAD];
+    over = __any(cnt > lst.cap);
+    u32 inc = cnt;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const u32 v = (u32)__shfl_up((int)inc, o, 64);
+      if (lane >= o) inc += v;
+    }
+    excl = inc - cnt;
+    total = (u32)__shfl((int)inc, 63, 64);
+    cap = lst.cap;
+  }
+  // where entry e lies; called by whole waves (the shuffles read all lanes)
+  __device__ __forceinline__ u64 at(u32 e) const
+  {
+    int sub = 0;
+#pragma unroll
+    for (int step = 32; step > 0; step >>= 1)
+      if ((u32)__shfl((int)excl, sub + step, 64) <= e) sub += step;
+    return (u64)sub * cap + (e - (u32)__shfl((int)excl, sub, 64));
+  }
+};
 
+// asym: the list is a folded k_pgather's unless *asym (null: not folded): a listed
+// chunk's gain counts for its block and, off the diagonal, for the block of its
+// row's sources too, whose mirrored chunks gain the same pairs.
 __global__ __launch_bounds__(LEVEL_WG) void k_sparse(const LevelTask* __restrict__ tasks, int ntasks,
-                                                     int level, int ring, LvList lst)
+                                                     int level, int ring, LvList lst, const u32* asym)
 {
+  const bool fold = asym && __builtin_amdgcn_readfirstlane(*asym) == 0;
   const u32 tid = blockIdx.x * blockDim.x + threadIdx.x, nth = gridDim.x * blockDim.x;
   const int lane = threadIdx.x & 63;
   // per running task: the count of level L starts from L-1's (slot L was
@@ -1008,36 +1272,23 @@ __global__ __launch_bounds__(LEVEL_WG) void k_sparse(const LevelTask* __restrict
     atomicAdd(&T.cnt[(int64_t)(level % ring) * T.cstride], T.cnt[(int64_t)((level - 1) % ring) * T.cstride]);
   }
   const u32 wbase = tid & ~63u;                       // the wave's first thread; loops are wave-uniform
-  // lane s holds sub-list s's count (LIST_SUBS is the wave size) and the
-  // count of the sub-lists before it: the sub-lists read as one list of
-  // `total` entries, entry e in the last sub-list starting at or below e
-  static_assert(LIST_SUBS == 64, "one sub-list per lane");
-  const u32 cnt = lst.n[lane * LIST_PAD];
-  if (!__any(cnt > lst.cap)) {
-    u32 inc = cnt;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const u32 v = (u32)__shfl_up((int)inc, o, 64);
-      if (lane >= o) inc += v;
-    }
-    const u32 excl = inc - cnt, total = (u32)__shfl((int)inc, 63, 64);
+  const ListView lv(lst, lane);
+  if (!lv.over) {
     // A task that stops at this level gains nothing: it stops because level
     // L-1 reached every pair (nothing listed) or added no bit (no chunk can
     // gain one now), so its listed chunks need no test.
-    for (u32 b = wbase; b < total; b += nth) {
+    for (u32 b = wbase; b < lv.total; b += nth) {
       const u32 e = b + lane;
-      int sub = 0;                                  // every lane searches (the shuffles read all lanes)
-#pragma unroll
-      for (int step = 32; step > 0; step >>= 1)
-        if ((u32)__shfl((int)excl, sub + step, 64) <= e) sub += step;
-      const u32 at = e - (u32)__shfl((int)excl, sub, 64);
-      int t = 0, gain = 0;
-      if (e < total) {
-        const u64 v = lst.e[(u64)sub * lst.cap + at];
+      const u64 k = lv.at(e);
+      int t = 0, t2 = 0, gain = 0;
+      if (e < lv.total) {
+        const u64 v = lst.e[k];
         t = (int)(v >> 48);
+        t2 = (int)((v >> 24) & 0xffffff) / PG_UNIT;
         gain = chunk_gain(tasks[t], level, (int)((v >> 24) & 0xffffff), (int)(v & 0xffffff));
       }
       add_gains(tasks, level, ring, t, gain);
+      if (fold) add_gains(tasks, level, ring, t2, t2 == t ? 0 : gain);
     }
   } else {
     for (int t = 0; t < ntasks; t++) {
@@ -1051,6 +1302,150 @@ __global__ __launch_bounds__(LEVEL_WG) void k_sparse(const LevelTask* __restrict
         if (i < total) gain = chunk_gain(T, level, (int)(i / chunks), 2 * (int)(i % chunks));
         add_gains(tasks, level, ring, t, gain);
       }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Thin levels.  When a level L is expected to leave hardly a pair (the level
+// after it the last), most of its gathers find their chunk saturated: at
+// n = 65536, d = 16 level 4 meets rows 59 % full, and twelve of a row's sixteen
+// neighbours fill 99.6 % of the chunks.  So k_pgather takes those neighbours
+// alone (LV_THIN) and lists the chunks left unsaturated with their bits; k_thin
+// completes the listed chunks from the rows' other neighbours; and level L + 1 is
+// done by k_thin2 from level L - 1's rows, two steps away, for the few chunks
+// still unsaturated.  Level L's rows are never written.  The counts are all pairs
+// less what the listed chunks still miss.  When the guess is wrong the host
+// stores levels L and L + 1 (their counts stand); when a list overflows, both
+// kernels leave the counts alone and k_thin2 marks level L + 1 (THIN_FAILED) for the
+// host, which runs level L whole.  n = 65536, d = 16: a folded level 4 of 459 us
+// and k_sparse's 30 become 310 of k_pgather, 24 of k_thin and 26 of k_thin2.
+#define THIN_FAILED (~0ULL)
+
+__device__ __forceinline__ bool chunk_full(const u64x2& x, u64 f0, u64 f1) { return x.x == f0 && x.y == f1; }
+
+// all pairs of every running task, into its count of the level (a slot that is
+// zero), from which k_thin and k_thin2 take the missing ones
+__device__ __forceinline__ void thin_counts(const LevelTask* __restrict__ tasks, int ntasks, int level, int ring,
+                                            u32 tid, u32 nth, bool clear_next)
+{
+  for (u32 t = tid; t < (u32)ntasks; t += nth) {
+    const LevelTask& T = tasks[t];
+    if (*T.done) continue;
+    if (task_stops(T, level, ring)) { *T.done = 1; continue; }
+    if (clear_next) T.cnt[(int64_t)((level + 1) % ring) * T.cstride] = 0;
+    atomicAdd(&T.cnt[(int64_t)(level % ring) * T.cstride], (u64)T.n * (u64)T.l);
+  }
+}
+
+// the listed chunks completed; those still unsaturated counted as missing and
+// listed in lst2
+__global__ __launch_bounds__(LEVEL_WG) void k_thin(const LevelTask* __restrict__ tasks, int ntasks, int level,
+                                                   int ring, LvList lst, LvList lst2, const u32* asym, int cut)
+{
+  const bool fold = asym && __builtin_amdgcn_readfirstlane(*asym) == 0;
+  const u32 tid = blockIdx.x * blockDim.x + threadIdx.x, nth = gridDim.x * blockDim.x;
+  const int lane = threadIdx.x & 63;
+  const u32 wbase = tid & ~63u;
+  const ListView lv(lst, lane);
+  if (lv.over) return;                                // uniform
+  thin_counts(tasks, ntasks, level, ring, tid, nth, false);
+  for (u32 b = wbase; b < lv.total; b += nth) {       // wave-uniform
+    const u32 e = b + lane;
+    const u64 k = lv.at(e);
+    int t = 0, t2 = 0, miss = 0;
+    u64 id = 0;
+    u64x2 x;
+    x.x = x.y = 0;
+    bool unsat = false;
+    if (e < lv.total) {
+      id = lst.e[k];
+      x = lst.v[k];
+      t = (int)(id >> 48);
+      const int r = (int)((id >> 24) & 0xffffff), w = (int)(id & 0xffffff);
+      t2 = r / PG_UNIT;
+      const LevelTask& T = tasks[t];
+      const u64* __restrict__ cur = ((level & 1) ? T.buf1 : T.buf0) + w;
+      const u64 f0 = full_word(T.l, w), f1 = full_word(T.l, w + 1);
+      const int* nb = T.nbr + (int64_t)r * T.dpad;
+      // the row's ids from `cut` on first: the thin pairs are its first ones in
+      // the order of the parts.  Sixteen ids at a time, their reads in flight
+      // together (one id group after the other took 116 us for 100 k chunks)
+      for (int pass = 0; pass < 2 && !chunk_full(x, f0, f1); pass++)
+        for (int j = 0; j < T.dpad && !chunk_full(x, f0, f1); j += 16) {
+          int4 q[4];
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            q[i] = make_int4(r, r, r, r);
+            if (j + 4 * i < T.dpad) q[i] = *(const int4*)(nb + j + 4 * i);
+          }
+          u64x2 o[16];
+#pragma unroll
+          for (int i = 0; i < 16; i++) {
+            const int v = i % 4 == 0 ? q[i / 4].x : i % 4 == 1 ? q[i / 4].y : i % 4 == 2 ? q[i / 4].z : q[i / 4].w;
+            o[i].x = o[i].y = 0;
+            if ((v >= cut) == (pass == 0) && v != r) o[i] = *(const u64x2*)(cur + (int64_t)v * 16);
+          }
+#pragma unroll
+          for (int i = 0; i < 16; i++) { x.x |= o[i].x; x.y |= o[i].y; }
+        }
+      miss = __popcll(f0 & ~x.x) + __popcll(f1 & ~x.y);
+      unsat = miss != 0;
+    }
+    add_gains(tasks, level, ring, t, -miss);
+    if (fold) add_gains(tasks, level, ring, t2, t2 == t ? 0 : -miss);
+    list_append(lst2, unsat, id, x.x, x.y);
+  }
+}
+
+// level L + 1 (`level`) from level L - 1's rows: a wave per chunk of lst2, its lanes
+// over the pairs of a neighbour and a neighbour's neighbour
+__global__ __launch_bounds__(LEVEL_WG) void k_thin2(const LevelTask* __restrict__ tasks, int ntasks, int level,
+                                                    int ring, LvList lst, LvList lst2, const u32* asym)
+{
+  const bool fold = asym && __builtin_amdgcn_readfirstlane(*asym) == 0;
+  const u32 tid = blockIdx.x * blockDim.x + threadIdx.x, nth = gridDim.x * blockDim.x;
+  const int lane = threadIdx.x & 63;
+  const ListView la(lst, lane), lv(lst2, lane);
+  if (la.over || lv.over) {                           // uniform
+    if (tid == 0) tasks[0].cnt[(int64_t)(level % ring) * tasks[0].cstride] = THIN_FAILED;
+    return;
+  }
+  thin_counts(tasks, ntasks, level, ring, tid, nth, true);
+  const u32 nwaves = nth >> 6;
+  for (u32 e = __builtin_amdgcn_readfirstlane(tid >> 6); e < lv.total; e += nwaves) {
+    const u64 k = lv.at(e);                           // the same in every lane
+    const u64 id = lst2.e[k];
+    const u64x2 x0 = lst2.v[k];
+    const int t = (int)(id >> 48), r = (int)((id >> 24) & 0xffffff), w = (int)(id & 0xffffff);
+    const LevelTask& T = tasks[t];
+    const u64* __restrict__ cur = ((level & 1) ? T.buf0 : T.buf1) + w;   // what level L read
+    const int* __restrict__ nbr = T.nbr;
+    const int dp = T.dpad, m = dp * (dp + 1);
+    u64x2 x = x0;
+    for (int i0 = lane; i0 < m; i0 += 64 * 4) {       // four pairs a lane in flight (past the last: the chunk's own row)
+      int u[4], q[4], v[4];
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const int i = i0 + 64 * c, j = i / (dp + 1);
+        q[c] = i < m ? i - j * (dp + 1) : dp;
+        u[c] = nbr[(int64_t)r * dp + (i < m ? j : 0)];
+      }
+#pragma unroll
+      for (int c = 0; c < 4; c++) v[c] = nbr[(int64_t)u[c] * dp + (q[c] == dp ? 0 : q[c])];
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const u64x2 o = *(const u64x2*)(cur + (int64_t)(q[c] == dp ? u[c] : v[c]) * 16);
+        x.x |= o.x; x.y |= o.y;
+      }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) { x.x |= __shfl_xor(x.x, o, 64); x.y |= __shfl_xor(x.y, o, 64); }
+    const int miss = __popcll(full_word(T.l, w) & ~x.x) + __popcll(full_word(T.l, w + 1) & ~x.y);
+    const int t2 = r / PG_UNIT;
+    if (lane == 0 && miss) {
+      atomicAdd(&T.cnt[(int64_t)(level % ring) * T.cstride], 0 - (u64)miss);
+      if (fold && t2 != t) atomicAdd(&tasks[t2].cnt[(int64_t)(level % ring) * T.cstride], 0 - (u64)miss);
     }
   }
 }
