@@ -33,7 +33,12 @@
 
 static const int KIND_MATRIX = 1, KIND_SAVING = 2, KIND_BFS = 3;   // the reference's ASPL_* (common.h:39-41)
 static const int GPU_CHUNK_WORDS = 64;          // column-block width of MATRIX_SAVING (parameter.h:13)
-static const int SAVING_GROUP = 32;             // MATRIX_SAVING blocks resident at once (4 per XCD)
+static const int SAVING_GROUP = 32;             // MATRIX_SAVING blocks resident at once (4 per XCD) ...
+static const size_t SAVING_BYTES = 16ull << 30;  // ... unless all blocks' buffers stay within this (and half the free
+                                                // memory): the folded levels need them all resident, and k_direct
+                                                // walks the rows once instead of once per group (n = 100000, d = 8:
+                                                // 4.99 -> 3.28 ms; n = 131072, d = 16: 10.8 -> 6.5 ms; n = 200000,
+                                                // d = 8, 10 GB: 28.4 -> 17.2 ms)
 static const int LEVEL_BLOCK_WORDS = 16;        // default column-block width of the level plan
 static const int RES_WB_MAX = 8;                // widest resident block: 256 sources
 static const int BATCH_CLASSES = 5;             // size classes of the batch launch policy
@@ -848,6 +853,11 @@ struct Evaluator {
     return d_xy2row && dpad <= 16 && 4 * ntiles <= n && !ext_adj;
   }
 
+  int parts_default(int kw) const
+  {
+    return kw == LEVEL_BLOCK_WORDS && (n >= PG_MIN_ROWS || (n >= PG_MIN_ROWS_NARROW && dpad <= 16)) ? PG_PARTS : 0;
+  }
+
   ODPX_Plan default_plan(int kind) const
   {
     ODPX_Plan p{};
@@ -887,8 +897,12 @@ struct Evaluator {
     // (measured against k_level at n = 16386-28000, d = 8, 16, 32: from n = 24576 the
     // part gather is 4-30 % faster at every degree but one (28000, d = 32: 2 % slower);
     // at n = 20000 it is 11-22 % faster for d <= 16 and 5 % slower for d = 32)
-    p.parts = (p.kw == LEVEL_BLOCK_WORDS && (n >= PG_MIN_ROWS || (n >= PG_MIN_ROWS_NARROW && dpad <= 16)))
-                  ? PG_PARTS : 0;
+    p.parts = parts_default(p.kw);
+    if (p.group && p.parts && s == 1) {
+      const size_t bytes = (size_t)((W + p.kw - 1) / p.kw) * 2 * n * p.kw * 8;
+      size_t avail = 0, total = 0;
+      if (bytes <= SAVING_BYTES && hipMemGetInfo(&avail, &total) == hipSuccess && bytes <= avail / 2) p.group = 0;
+    }
     if (tile_capable()) {
       // grid graphs: 2-word blocks and temporal tiles (k_tile); MATRIX_SAVING
       // keeps the same number of source words resident as with 16-word blocks
@@ -1259,7 +1273,7 @@ struct Evaluator {
   // whether the level before a count-only level `spec` lists its unsaturated chunks
   bool listed_at(int spec) const
   {
-    return !lv.fr && list_ok() && spec - 1 >= lv.L1 && lr.ntasks < 65536 && n < (1 << 24) && lr.kwp < (1 << 24);
+    return spec >= 0 && !lv.fr && list_ok() && spec - 1 >= lv.L1 && lr.ntasks < 65536 && n < (1 << 24) && lr.kwp < (1 << 24);
   }
 
   // gather levels [from, to) of the current group, then the counter and error copies.
@@ -1273,7 +1287,7 @@ struct Evaluator {
       lv_copies(to);
       return;
     }
-    const bool listed = listed_at(lv.spec);
+    const bool listed = listed_at(lv.spec) && from < lv.spec;   // the level before it is in this batch
     for (int L = from; L < to; L++) {
       int mode = LV_STORE | LV_COUNT;
       if (L == lv.spec) mode = listed ? LV_SPARSE : LV_COUNT;
@@ -1449,7 +1463,14 @@ struct Evaluator {
   {
     if (lv.tk) return tile_batch_end(lv.L1, guess_levels > 0 ? guess_levels - lv.L1 : 8);
     const int be = std::min(n, std::max(2, std::min(MAX_BATCH_LEVELS, guess_levels > 0 ? guess_levels : 8)));
-    return std::min(be, std::max(lv.L1 + batch_cap, 2));
+    return capped_end(std::min(be, std::max(lv.L1 + batch_cap, 2)));
+  }
+
+  // a batch cut short (serving) that would end one level before the expected
+  // last one takes that level too: the two run listed (thin) and sparse
+  int capped_end(int be) const
+  {
+    return batch_cap < MAX_BATCH_LEVELS && be == guess_levels - 1 && be - 1 >= lv.L1 ? guess_levels : be;
   }
 
   // tile mode: batches are whole launches of lv.tk levels, short enough that
@@ -1598,7 +1619,11 @@ struct Evaluator {
     }
     if (lv.running > 0 && lv.launched < n) {
       const int step = std::min(batch_cap, std::min(MAX_BATCH_LEVELS, std::max(lv.launched, 8)));
-      lv.batch_end = lv.tk ? tile_batch_end(lv.launched, step) : std::min(n, lv.launched + step);
+      lv.batch_end = lv.tk ? tile_batch_end(lv.launched, step) : capped_end(std::min(n, lv.launched + step));
+      if (batch_cap < MAX_BATCH_LEVELS && spec_at(lv.batch_end)) {
+        lv.spec = lv.batch_end - 1;
+        lv.thin = lv.launched < lv.spec && listed_at(lv.spec) && pg_on() && thin_k > 0;
+      }
       lv_levels(lv.launched, lv.batch_end);
       lv.launched = std::max(lv.launched, lv.batch_end);
       return false;

@@ -92,6 +92,8 @@ struct SvChain {
   size_t bytes = 0;
   std::deque<long long> queue;      // pending requests, FIFO
   bool busy = false;                // its front request is in a slot
+  int guess = 0, thin_k = 0;        // what its last level-plan evaluation expects of the next
+  bool list_on = true;
 };
 
 struct SvReq {
@@ -261,11 +263,14 @@ static void sv_large_launch(SvLargeSlot& sl, int ci)
     ODPX_Plan p{};
     p.plan = ODPX_PLAN_LEVEL; p.kw = LEVEL_BLOCK_WORDS; p.upw = 8; p.seg_major = 0; p.xcd = 1; p.group = 0;
     p.direct = -1; p.batch = 0;
+    p.parts = ev.parts_default(std::min(LEVEL_BLOCK_WORDS, (c.n + 63) / 64));
     ev.apply_plan(p);
     sl.shaped_n = c.n; sl.shaped_d = c.degree;
   }
   ev.ext_adj = c.d_adj;
   ev.batch_cap = sv_large_levels();
+  // the chain's own level count and last levels, not the slot's last chain's
+  ev.guess_levels = c.guess; ev.list_on = c.list_on; ev.thin_k = c.thin_k;
   ev.lv_begin();
   HIPC(hipEventRecord(sl.done, ev.st));
   sl.busy = true;
@@ -294,6 +299,8 @@ static void sv_large_advance(SvLargeSlot& sl)
     r.diameter = d; r.sum = sm; r.aspl = as;
     r.status = *sl.h_status ? -1 : 0;
   }
+  SvChain& c = S.chains[sl.chain];
+  c.guess = ev.guess_levels; c.list_on = ev.list_on; c.thin_k = ev.thin_k;
   r.t_done = mono_time();
   sv_complete(sl.id);
   sl.busy = false;
