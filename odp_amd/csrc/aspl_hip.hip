@@ -170,10 +170,9 @@ static void ctx_init()
   HIPC(hipFuncSetAttribute((const void*)k_anneal<2>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_DYN_MAX));
   HIPC(hipFuncSetAttribute((const void*)k_anneal<4>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_DYN_MAX));
   HIPC(hipFuncSetAttribute((const void*)k_anneal<8>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_DYN_MAX));
-  HIPC(hipFuncSetAttribute((const void*)k_direct<true, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_DYN_MAX));
-  HIPC(hipFuncSetAttribute((const void*)k_direct<true, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_DYN_MAX));
-  HIPC(hipFuncSetAttribute((const void*)k_direct<false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_DYN_MAX));
-  HIPC(hipFuncSetAttribute((const void*)k_direct<false, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_DYN_MAX));
+  for (auto k : {k_direct<true, true, true>, k_direct<true, false, true>, k_direct<true, false, false>,
+                 k_direct<false, true, false>, k_direct<false, false, false>})
+    HIPC(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_DYN_MAX));
   C.ready = true;
   trace("ctx ready");
 }
@@ -946,17 +945,30 @@ struct Evaluator {
     for (int i = 0; i <= K; i++) { t += m; m *= dpad; if (m > (1L << 40)) m = 1L << 40; }
     return t;
   }
-  // ints of walk-tree ids k_direct keeps per wave: 4 for depth 0, dpad^d for 0 < d < K
-  long direct_list(int K) const
+  // ints k_direct's depth lists take per wave.  A launch over every source (all)
+  // keeps breadth-first frontiers, at most degree^d ids at depth d, 16 bits each
+  // when they fit; the others whole walk trees: 4 ints for depth 0, dpad^d for 0 < d < K
+  long direct_list(int K, bool all) const
   {
-    long t = 4, m = 1;
-    for (int i = 1; i < K; i++) { m *= dpad; t += m; }
-    return t;
+    long t = all ? 1 : 4, m = 1;
+    for (int i = 1; i < K; i++) { m *= all ? std::max(degree, 1) : dpad; t += m; }
+    return all && n <= 65536 ? (t + 1) / 2 : t;
+  }
+  // every source in one launch of `group` blocks of kw words
+  bool direct_all(int kw, int group) const
+  {
+    return src_lo == 0 && src_hi == n && (int64_t)group * kw * 64 >= n;
+  }
+  void (*direct_kernel(int kw, int group) const)(DirectArgs)
+  {
+    const bool id16 = direct16();
+    if (!direct_all(kw, group)) return id16 ? k_direct<false, true, false> : k_direct<false, false, false>;
+    return id16 ? k_direct<true, true, true> : n <= 65536 ? k_direct<true, false, true> : k_direct<true, false, false>;
   }
   size_t direct_lds(int K, int kw, int group, int nw) const
   {
     const size_t words = (size_t)group * kw, chunks = (words + 127) / 128;
-    return (size_t)nw * (words * 8 + (size_t)direct_list(K) * 4) + (size_t)K * chunks * 64 * 4;
+    return (size_t)nw * (words * 8 + (size_t)direct_list(K, direct_all(kw, group)) * 4) + (size_t)K * chunks * 64 * 4;
   }
   // waves per workgroup k_direct can run with (0: not applicable): the block
   // rows must be a power of two of 2..128 words and one row bitmap must fit
@@ -1073,10 +1085,18 @@ struct Evaluator {
     if (r.direct >= n) r.direct = 0;
     plan.direct = r.direct;            // the plan reports the K that runs
     if (r.direct) {
+      // Over every source: the largest workgroup, up to 16 waves, that LDS holds --
+      // every workgroup adds its counts with an atomic per block and level, so few
+      // large ones beat more waves in small ones (n = 28000, d = 16: 16 waves 74 us,
+      // 2 x 8 80, 2 x 10 93, 5 x 4 102, 20 x 1 240; n = 100000, d = 8: 10 waves).
       r.dnw = direct_waves(r.direct, kw, group);
+      if (direct_all(kw, group))
+        for (int nw = 16; nw >= 1; nw--)
+          if (direct_lds(r.direct, kw, group, nw) <= LDS_DYN_MAX) { r.dnw = nw; break; }
       r.dlds = direct_lds(r.direct, kw, group, r.dnw);
-      int per_cu = (int)std::max<size_t>(1, LDS_LIMIT / r.dlds);
-      per_cu = std::min(per_cu, 32 / r.dnw);
+      int per_cu = 0;
+      HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, direct_kernel(kw, group), 64 * r.dnw, r.dlds));
+      per_cu = std::max(1, std::min(per_cu, 32 / r.dnw));
       r.dgrid = std::max(1, std::min((n + r.dnw - 1) / r.dnw, per_cu * C.ncu));
     }
     std::vector<LevelTask> ht(ntasks);
@@ -1248,7 +1268,7 @@ struct Evaluator {
       a.src_lo = src_lo + first * r.kw * 64;
       a.nsrc = std::min(cnt_t * r.kw * 64, src_hi - a.src_lo);
       a.ntask = cnt_t; a.words = cnt_t * r.kw; a.chunks = (a.words + 127) / 128;
-      a.K = K; a.list = (int)direct_list(K);
+      a.K = K; a.list = (int)direct_list(K, direct_all(r.kw, r.group));
       // streamed stores when the row-part gather reads the rows next (measured: n=65536
       // 591 -> 600 evaluations/s); the tile plan re-reads them soon (the grid ran 2.7 % slower)
       a.nt = pg_on() ? 1 : 0;
@@ -1258,10 +1278,7 @@ struct Evaluator {
       a.qmul = q > 1 ? (unsigned)((1ULL << 32) / q + 1) : 0u;
       long m = 1;
       for (int i = 0; i < 8; i++) { a.pw[i] = (int)m; m = std::min<long>(m * dpad, 1L << 30); }
-      const bool all = a.src_lo == 0 && a.nsrc == n;
-      auto kern = all ? (id16 ? k_direct<true, true> : k_direct<true, false>)
-                      : (id16 ? k_direct<false, true> : k_direct<false, false>);
-      hipLaunchKernelGGL(kern, dim3(r.dgrid), dim3(64 * r.dnw), r.dlds, st, a);
+      hipLaunchKernelGGL(direct_kernel(r.kw, r.group), dim3(r.dgrid), dim3(64 * r.dnw), r.dlds, st, a);
     } else {
       hipLaunchKernelGGL(k_level0, dim3(cnt_t * r.per_task_wg), dim3(LEVEL_WG), 0, st,
                          r.tasks + first, r.wg_start, cnt_t, RING, r.upw, r.xcd);

@@ -28,6 +28,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 typedef unsigned long long u64;
 typedef unsigned int u32;
@@ -1755,6 +1756,14 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile(const LevelTask* __restri
 // written to the buffer level K reads.  The sets are exactly those the level
 // kernels build, so every count and every word equals k_level0 followed by
 // levels 1..K-1.
+//
+// A launch over every source (ALL) drops the ids its bitmap already holds: the
+// walks on from a vertex met before end where its first occurrence's end, so a
+// depth's list is the breadth-first frontier (485 instead of 1365 expanded ids
+// at d = 4, K = 6), its length the level's count, and only the last depth's
+// bitmap is popcounted.  Bound by LDS atomics and the latency of a row's K
+// dependent table reads.  n = 49999, d = 4: 332 -> 135 us; n = 100000, d = 8:
+// 678 -> 389; n = 65536, d = 16 (4112 of 4368 ids): 170 -> 147.
 
 struct DirectArgs {
   const int* nbr;        // [n][dpad] row-neighbour table
@@ -1768,7 +1777,7 @@ struct DirectArgs {
   int ntask, words;      // blocks in the group; words = ntask * kw
   int chunks;            // ceil(words / 128): 128-word chunks a wave sweeps per row
   int K;                 // levels computed (2..DIRECT_KMAX)
-  int list;              // ints of walk-tree ids kept per wave: 4 + sum of dpad^i, 0 < i < K
+  int list;              // ints a wave's depth lists take (Evaluator::direct_list)
   unsigned qmul;         // floor(2^32 / q) + 1 for q = 16-byte loads per table row > 1:
                          // idx / q == umulhi(idx, qmul) for idx < 2^32 / q (idx < 2^24, q <= 256 here)
   int pw[8];             // dpad^i
@@ -1777,6 +1786,7 @@ struct DirectArgs {
 
 #define DIRECT_KMAX 6
 #define DIRECT_UNROLL 8
+#define DIRECT_UNROLL_BFS 4
 
 // ALL: every id is a source of the group (src_lo == 0, nsrc == n), no range test
 template <bool ALL>
@@ -1787,8 +1797,9 @@ __device__ __forceinline__ void direct_set(u32* bm, int id, int src_lo, int nsrc
 }
 
 // ID16: the 16-bit table (eight ids per 16-byte load) instead of the 32-bit one
-template <bool ALL, bool ID16>
-__global__ __launch_bounds__(512) void k_direct(DirectArgs a)
+// L16: the depth lists hold 16-bit ids (ALL, n <= 65536): less LDS, more waves
+template <bool ALL, bool ID16, bool L16>
+__global__ __launch_bounds__(1024) void k_direct(DirectArgs a)
 {
   extern __shared__ __attribute__((aligned(16))) u64 dlds[];
   const int nw = blockDim.x >> 6;
@@ -1800,7 +1811,9 @@ __global__ __launch_bounds__(512) void k_direct(DirectArgs a)
   // the workgroup (lane l of chunk j holds words 128 j + 2 l, 128 j + 2 l + 1).
   // Depth 0 takes 4 ints of a list and depth d >= 1 dpad^d, so every depth
   // starts 16-byte aligned (dpad is a multiple of 4).
-  int* list = (int*)(dlds + (int64_t)nw * a.words) + wave * a.list;
+  static_assert(ALL || !L16, "16-bit depth lists");
+  typedef typename std::conditional<L16, unsigned short, int>::type lid;
+  lid* list = (lid*)((int*)(dlds + (int64_t)nw * a.words) + wave * a.list);
   u32* lc = (u32*)((int*)(dlds + (int64_t)nw * a.words) + nw * a.list);
   const int ncnt = a.K * a.chunks * 64;
   for (int i = threadIdx.x; i < ncnt; i += blockDim.x) lc[i] = 0;
@@ -1813,16 +1826,71 @@ __global__ __launch_bounds__(512) void k_direct(DirectArgs a)
   // enough and the waves of a workgroup never wait for each other.
   for (int v = blockIdx.x * nw + wave; v < a.n; v += gridDim.x * nw) {   // wave-uniform
     for (int w = 2 * lane; w < a.words; w += 128) { u64x2 z; z.x = 0; z.y = 0; *(u64x2*)(bm + w) = z; }
-    if (lane == 0) list[0] = v;
+    if (lane == 0) list[0] = (lid)v;
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     if (lane == 0) direct_set<ALL>(bm32, v, a.src_lo, a.nsrc);
-    int off = 0;                                   // start of the depth d-1 list
-    for (int d = 1; d <= a.K; d++) {
-      const int m = a.pw[d - 1];                   // ids at depth d-1
+    int off = 0, m_last = 0;                       // start of the depth d-1 list; its ids (ALL, d = K)
+    if (ALL) {
+      // the bitmap holds every id, so it tells a new id from one met before,
+      // whose walks on from here end where its first occurrence's do: the depth
+      // lists are breadth-first frontiers, and their entries the level's count
+      if (lane == 0) atomicAdd(&lc[v >> 7], 1u);
+      int m = 1;
+      for (int d = 1; d < a.K; d++) {
+        const int jobs = m * Q;
+        const lid* from = list + off;
+        lid* to = list + off + m;
+        u32* lcd = lc + (d - 1) * a.chunks * 64;
+        int got = 0;                               // ids appended (uniform)
+        for (int j0 = 0; j0 < jobs; j0 += 64 * DIRECT_UNROLL_BFS) {
+          uint4 q[DIRECT_UNROLL_BFS];
+#pragma unroll
+          for (int u = 0; u < DIRECT_UNROLL_BFS; u++) {
+            const unsigned idx = j0 + u * 64 + lane;
+            if (idx < (unsigned)jobs) {
+              const unsigned r = Q == 1 ? idx : __umulhi(idx, a.qmul);
+              const int64_t e = (int64_t)from[r] * a.dpad + IPL * (idx - r * Q);
+              q[u] = ID16 ? *(const uint4*)(a.nbr16 + e) : *(const uint4*)(a.nbr + e);
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < DIRECT_UNROLL_BFS; u++) {
+            if (j0 + u * 64 < jobs) {              // uniform
+              const bool act = j0 + u * 64 + lane < jobs;
+              const u32 w4[4] = {q[u].x, q[u].y, q[u].z, q[u].w};
+              int id[ID16 ? 8 : 4];
+              u32 old[ID16 ? 8 : 4];
+#pragma unroll
+              for (int i = 0; i < (ID16 ? 8 : 4); i++) {
+                id[i] = ID16 ? (int)(i & 1 ? w4[i >> 1] >> 16 : w4[i >> 1] & 0xffff) : (int)w4[i];
+                old[i] = ~0u;
+                if (act) old[i] = atomicOr(&bm32[id[i] >> 5], 1u << (id[i] & 31));
+              }
+#pragma unroll
+              for (int i = 0; i < (ID16 ? 8 : 4); i++) {
+                const bool fresh = !((old[i] >> (id[i] & 31)) & 1);
+                const u64 mask = __ballot(fresh);
+                if (fresh) {
+                  to[got + __popcll(mask & ((1ULL << lane) - 1))] = (lid)id[i];
+                  atomicAdd(&lcd[id[i] >> 7], 1u);
+                }
+                got += __popcll(mask);
+              }
+            }
+          }
+        }
+        off += m;
+        m = got;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      }
+      m_last = m;
+    }
+    for (int d = ALL ? a.K : 1; d <= a.K; d++) {
+      const int m = ALL ? m_last : a.pw[d - 1];    // ids at depth d-1
       const int jobs = m * Q;
-      const int* from = list + off;
+      const lid* from = list + off;
       const int step = d == 1 ? 4 : m;             // ints the depth d-1 list takes
-      int* to = list + off + step;                 // the depth-d list follows
+      lid* to = list + off + step;                 // the depth-d list follows
       for (int j0 = 0; j0 < jobs; j0 += 64 * DIRECT_UNROLL) {
         uint4 q[DIRECT_UNROLL];
 #pragma unroll
@@ -1850,7 +1918,7 @@ __global__ __launch_bounds__(512) void k_direct(DirectArgs a)
               direct_set<ALL>(bm32, hi.y, a.src_lo, a.nsrc);
               direct_set<ALL>(bm32, hi.z, a.src_lo, a.nsrc);
               direct_set<ALL>(bm32, hi.w, a.src_lo, a.nsrc);
-              if (d < a.K) { *(int4*)(to + 8 * idx) = lo; *(int4*)(to + 8 * idx + 4) = hi; }
+              if (!ALL && d < a.K) { *(int4*)(to + 8 * idx) = lo; *(int4*)(to + 8 * idx + 4) = hi; }
             } else {
               int4 v;
               v.x = (int)q[u].x; v.y = (int)q[u].y; v.z = (int)q[u].z; v.w = (int)q[u].w;
@@ -1858,7 +1926,7 @@ __global__ __launch_bounds__(512) void k_direct(DirectArgs a)
               direct_set<ALL>(bm32, v.y, a.src_lo, a.nsrc);
               direct_set<ALL>(bm32, v.z, a.src_lo, a.nsrc);
               direct_set<ALL>(bm32, v.w, a.src_lo, a.nsrc);
-              if (d < a.K) *(int4*)(to + 4 * idx) = v;
+              if (!ALL && d < a.K) *(int4*)(to + 4 * idx) = v;
             }
           }
         }
@@ -1893,6 +1961,8 @@ __global__ __launch_bounds__(512) void k_direct(DirectArgs a)
   for (int e = wave; e < a.K * a.chunks; e += nw) {            // wave-uniform
     const int L = e / a.chunks, j = e - L * a.chunks;
     u64 c = lc[e * 64 + lane];
+    if (ALL && L < a.K - 1)                                    // the ids first met at each depth so far
+      for (int i = 0; i < L; i++) c += lc[(i * a.chunks + j) * 64 + lane];
     for (int o = 1; o < half; o <<= 1) c += __shfl_xor(c, o, 64);
     const int w = 128 * j + 2 * lane;
     if (w < a.words && (lane & (half - 1)) == 0 && c)
