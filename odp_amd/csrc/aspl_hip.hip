@@ -69,6 +69,7 @@ static const double LV_SPIN_S = 20e-3;           // a level batch's wait watches
 static const int LVFIN_MAX = 4096;               // counters k_lvfin hands over (more: copies, faster than one workgroup's writes to host memory)
 static const int RING = 260;                    // per-level counter slots kept on the device
 static const int MAX_BATCH_LEVELS = 256;        // levels launched between two host reads (< RING - 2)
+static const size_t MALL_BYTES = 256u << 20;    // the last-level cache in front of HBM
 static const int PG_PARTS = 4;                  // row parts of the XCD-phased gather (2 MiB of a 65536-row slab)
 static const int PG_MIN_ROWS = 24576;           // ... used by default from this many rows (a 3 MiB slab),
 static const int PG_MIN_ROWS_NARROW = 20000;    // ... and from this many with tables of at most 16 ids
@@ -249,16 +250,6 @@ static int res_width(int n, int nsrc, int wbmax, int ncu)
   return wb;
 }
 
-// cache policy of k_pgather's gathers (env ODP_HIP_PG_AUX: 0 default, 1 sc0, 16 sc1, 2 nt)
-static int pg_aux_env()
-{
-  const char* v = getenv("ODP_HIP_PG_AUX");
-  const int a = v ? atoi(v) : 0;
-  return (a == 1 || a == 16 || a == 2) ? a : 0;
-}
-
-// the share of unsaturated chunks up to which a count-only last level lists
-// them (env ODP_HIP_LIST_FRAC; a large value always lists)
 // ODP_HIP_FOLD=0: every unit of a gather level, whatever the table (diagnostics)
 static bool pg_fold_env()
 {
@@ -289,6 +280,8 @@ static int pg_cut(double units, double extra, int wgs)
   return best;
 }
 
+// the share of unsaturated chunks up to which a count-only last level lists
+// them (env ODP_HIP_LIST_FRAC; a large value always lists)
 static double list_frac_env(double dflt)
 {
   const char* v = getenv("ODP_HIP_LIST_FRAC");
@@ -379,7 +372,7 @@ struct LevelRun {
   u64* h_acnt = nullptr;                // processed-unit counts on the host (kernel timing only)
   size_t flag_bytes = 0;
   // part-phased gather (k_pgather): row parts, sorted neighbour runs, persistent grid
-  int parts = 0, psp = 0, pgrid = 0, pupt = 0, paux = 0;
+  int parts = 0, psp = 0, pgrid = 0, pupt = 0;
   bool fold = false;                    // folded levels where the table is symmetric (k_pgather)
   int cut_full = 0, cut_fold = 0;       // log2 of the pieces its last round's units are cut into
   u32* plist = nullptr; int* ppoff = nullptr;  // per unit of PG_UNIT rows: pairs grouped by part, offsets
@@ -935,6 +928,8 @@ struct Evaluator {
   // gather levels run k_pgather: a plan with parts, plain (not frontier, not tile) levels
   bool pg_on() const { return plan.plan == ODPX_PLAN_LEVEL && lr.parts > 0 && !lv.fr && !lv.tk; }
   // k_direct reads the 16-bit table when it exists with the 32-bit table's width
+  // whether the gather levels' rows are streamed: the resident blocks' two buffers pass the last-level cache
+  int pg_streamed() const { return (size_t)lr.group * 2 * n * lr.kwp * 8 > MALL_BYTES ? 1 : 0; }
   bool direct16() const
   {
     return plan.plan == ODPX_PLAN_LEVEL && lr.direct > 0 && d_nbr16 && dp16 == dpad;
@@ -1060,15 +1055,14 @@ struct Evaluator {
       const size_t nl = (size_t)r.pupt * PG_UNIT * r.psp, np = (size_t)r.pupt * PG_OFF;
       if (nl > r.plist_cap) { dfree(&r.plist); dalloc(&r.plist, nl); r.plist_cap = nl; }
       if (np > r.ppoff_cap) { dfree(&r.ppoff); dalloc(&r.ppoff, np); r.ppoff_cap = np; }
-      r.paux = pg_aux_env();
       if (!r.list_v) {
         dalloc(&r.list_v, (size_t)THIN_CAP);
         dalloc(&r.list2, (size_t)THIN2_CAP); dalloc(&r.list2_v, (size_t)THIN2_CAP);
       }
       // persistent grid: every workgroup the CUs hold at once, a multiple of the XCD count
       int occ = 0, occ_ls = 0;
-      HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_pgather<false, 0>, PG_WG, 0));
-      HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ_ls, k_pgather<true, 0>, PG_WG, 0));
+      HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_pgather<false, true>, PG_WG, 0));
+      HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ_ls, k_pgather<true, true>, PG_WG, 0));
       occ = std::max(1, std::min(occ, occ_ls));
       r.pgrid = ODP_NXCD * std::max(1, C.ncu / ODP_NXCD) * occ;
       // folded levels need the whole matrix resident, a task per PG_UNIT rows
@@ -1269,9 +1263,9 @@ struct Evaluator {
       a.nsrc = std::min(cnt_t * r.kw * 64, src_hi - a.src_lo);
       a.ntask = cnt_t; a.words = cnt_t * r.kw; a.chunks = (a.words + 127) / 128;
       a.K = K; a.list = (int)direct_list(K, direct_all(r.kw, r.group));
-      // streamed stores when the row-part gather reads the rows next (measured: n=65536
-      // 591 -> 600 evaluations/s); the tile plan re-reads them soon (the grid ran 2.7 % slower)
-      a.nt = pg_on() ? 1 : 0;
+      // streamed stores when the row-part gather reads the rows next, by its own rule (measured:
+      // n=65536 591 -> 600 evaluations/s); the tile plan re-reads them soon (the grid ran 2.7 % slower)
+      a.nt = pg_on() ? pg_streamed() : 0;
       const bool id16 = direct16();
       const unsigned q = (unsigned)(dpad / (id16 ? 8 : 4));
       a.nbr16 = d_nbr16;
@@ -1376,10 +1370,9 @@ struct Evaluator {
       a.asym = asym;
       a.cut_full = r.cut_full; a.cut_fold = r.cut_fold;
       const bool ls = (mode & LV_LIST) != 0;
-      auto kern = r.paux == 1 ? (ls ? k_pgather<true, 1> : k_pgather<false, 1>)
-                : r.paux == 16 ? (ls ? k_pgather<true, 16> : k_pgather<false, 16>)
-                : r.paux == 2 ? (ls ? k_pgather<true, 2> : k_pgather<false, 2>)
-                : (ls ? k_pgather<true, 0> : k_pgather<false, 0>);
+      const bool nt = pg_streamed() != 0;
+      auto kern = ls ? (nt ? k_pgather<true, true> : k_pgather<true, false>)
+                     : (nt ? k_pgather<false, true> : k_pgather<false, false>);
       hipLaunchKernelGGL(kern, dim3(r.pgrid), dim3(PG_WG), 0, st, r.tasks + lv.first, L, RING, mode, lst, a);
     } else {
       const bool ls = (mode & LV_LIST) != 0;
@@ -1521,7 +1514,9 @@ struct Evaluator {
     if (lv.check) {
       const int64_t total = (int64_t)n * dpad;
       const int grid = (int)std::min<int64_t>(std::max<int64_t>(1, (total + 255) / 256), 4096);
-      hipLaunchKernelGGL(k_symcheck, dim3(grid), dim3(256), 0, st, d_nbr, n, dpad, r.asym);
+      auto kern = dpad == 4 ? k_symcheck<1> : dpad == 8 ? k_symcheck<2> : dpad == 12 ? k_symcheck<3>
+                : dpad == 16 ? k_symcheck<4> : k_symcheck<0>;
+      hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, st, d_nbr, n, dpad, r.asym);
       HIPC(hipGetLastError());
     }
     if (pg_on() && !lv.plfresh) {

@@ -238,8 +238,10 @@ __global__ void k_swap(int* adj, int degree, int a, int b, int c, int d, int* er
 // Sets *asym unless the table is symmetric: row u holds row r as many times as
 // row r holds u (entries equal to the row itself are padding).  Counting the
 // repeats makes the property outlive 2-opt swaps: each removes and adds one
-// entry of both directions.  A thread per entry, 16 bytes a load: 41 -> 14 us at
-// n = 65536, d = 16 against a loop over single ids.
+// entry of both directions.  A thread per entry, 16 bytes a load, a row's loads
+// in flight together (Q of them; 0: any width): 12 us at n = 65536, d = 16, 21 with
+// the loads one after the other, 41 over single ids.
+template <int Q>
 __global__ void k_symcheck(const int* __restrict__ nbr, int n, int dpad, u32* asym)
 {
   const int64_t total = (int64_t)n * dpad;
@@ -252,10 +254,18 @@ __global__ void k_symcheck(const int* __restrict__ nbr, int n, int dpad, u32* as
     const int4* own = (const int4*)(nbr + (int64_t)r * dpad);
     const int4* his = (const int4*)(nbr + (int64_t)u * dpad);
     int c = 0;
-    for (int k = 0; k < dpad >> 2; k++) {
-      const int4 o = own[k], h = his[k];
+    auto add = [&](const int4& o, const int4& h) {
       c += (o.x == u) + (o.y == u) + (o.z == u) + (o.w == u);
       c -= (h.x == r) + (h.y == r) + (h.z == r) + (h.w == r);
+    };
+    if (Q) {
+      int4 o[Q ? Q : 1], h[Q ? Q : 1];
+#pragma unroll
+      for (int k = 0; k < Q; k++) { o[k] = own[k]; h[k] = his[k]; }
+#pragma unroll
+      for (int k = 0; k < Q; k++) add(o[k], h[k]);
+    } else {
+      for (int k = 0; k < dpad >> 2; k++) add(own[k], his[k]);
     }
     bad = bad || c != 0;
   }
@@ -855,15 +865,24 @@ __device__ __forceinline__ void lds_barrier()
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// A level's rows are streamed past the caches (nt) unless both levels' rows
+// fit the 256 MB last-level cache, from which the next level then gathers
+// (n = 30002, d = 16: an evaluation 281 -> 247 us; n = 65536: 952 streamed, 1026 not)
+template <bool NT>
+__device__ __forceinline__ void row_store(u64v2 o, u64v2* p)
+{
+  if (NT) __builtin_nontemporal_store(o, p);
+  else *p = o;
+}
+
 // Persistent: workgroup b runs on XCD b % 8 and takes every (gridDim.x / 8)-th
 // unit of its XCD's contiguous range of units (a unit: PG_UNIT rows of one
 // task), so the XCD's workgroups sweep that range together; any grid that is a
 // multiple of 8 works.  The units of the last round, when they do not fill it,
 // are cut into pieces of their rows (2^cut of them) dealt over the workgroups.
-// The gathers are buffer loads with cache policy AUX
-// (0: default; 1: sc0, 16: sc1, 2: nt), bounded by the slab (out-of-range
-// offsets read zero).
-template <bool LS, int AUX>
+// The gathers are buffer loads bounded by the slab (out-of-range offsets read
+// zero).  LS: listing; NT: rows streamed past the caches.
+template <bool LS, bool NT>
 __global__ __launch_bounds__(PG_WG) void k_pgather(const LevelTask* __restrict__ tasks, int level, int ring,
                                                    int mode, LvList lst, PgArgs a)
 {
@@ -992,7 +1011,7 @@ __global__ __launch_bounds__(PG_WG) void k_pgather(const LevelTask* __restrict__
       const u32 e = (u32)__shfl((int)chunk.v[q >> 3], (q & 7) * 8 + (lane >> 3), 64);
       lr[q] = e == SENT ? -1 : (int)(e >> 22);
       const u32 off = e == SENT ? 0xfffffff0u : (e & 0x3fffff) * 128u + w * 8u;
-      const u32x4v v = __builtin_amdgcn_raw_buffer_load_b128(src, (int)off, 0, AUX);
+      const u32x4v v = __builtin_amdgcn_raw_buffer_load_b128(src, (int)off, 0, 0);
       gv[q].x = ((u64)v.y << 32) | v.x; gv[q].y = ((u64)v.w << 32) | v.z;
     };
     const Pairs first = pairs(wave);
@@ -1043,7 +1062,7 @@ __global__ __launch_bounds__(PG_WG) void k_pgather(const LevelTask* __restrict__
         if (valid) {
           if (store) {
             u64v2 o; o.x = v.x; o.y = v.y;
-            __builtin_nontemporal_store(o, (u64v2*)(nxt + (int64_t)r * 16 + w));   // streamed past L2
+            row_store<NT>(o, (u64v2*)(nxt + (int64_t)r * 16 + w));
           }
           pop += (u64)(__popcll(v.x) + __popcll(v.y));
         }
@@ -1090,7 +1109,7 @@ __global__ __launch_bounds__(PG_WG) void k_pgather(const LevelTask* __restrict__
           const u64x2 v = acc[c * 8 + (kq ^ (f >> 1))];
           u64v2 o;
           o.x = f & 1 ? v.y : v.x; o.y = f & 1 ? v.x : v.y;
-          if (r < a.n) __builtin_nontemporal_store(o, (u64v2*)(mnxt + (int64_t)r * 16 + w));
+          if (r < a.n) row_store<NT>(o, (u64v2*)(mnxt + (int64_t)r * 16 + w));
         }
       }
       lds_barrier();                                // acc is free for the next unit
