@@ -426,8 +426,8 @@ extern "C" int ODPX_Serve_add_chain(int nodes, int degree, const int* adjacency)
     HIPC(hipMemcpy(d_g, &G, sizeof G, hipMemcpyHostToDevice));
     HIPC(hipMemset(d_err, 0, sizeof(int)));
     long long total = (long long)nodes * c.dp16;
-    hipLaunchKernelGGL(k_prepare_batch, dim3((int)std::min<long long>((total + 255) / 256, 4096)), dim3(256), 0, 0,
-                       d_g, 1, total, c.d_adj, c.d_nbr16, d_err);
+    hipLaunchKernelGGL(k_prepare_batch, dim3((int)std::min<long long>((total / 8 + 255) / 256, 4096)), dim3(256), 0, 0,
+                       d_g, 1, 0LL, total, c.d_adj, c.d_nbr16, d_err);
     HIPC(hipGetLastError());
     HIPC(hipMemcpy(&h_err, d_err, sizeof(int), hipMemcpyDeviceToHost));
     dfree(&d_g); dfree(&d_err);
