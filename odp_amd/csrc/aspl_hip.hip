@@ -1337,7 +1337,8 @@ struct Evaluator {
     if (j == 0) hipLaunchKernelGGL(k_clear, dim3(1), dim3(64), 0, st, (u64*)nullptr, 0, (int*)r.tq, 1);
     hipLaunchKernelGGL(k_tile_plan, dim3(std::min((units + 255) / 256, 1024)), dim3(256), 0, st,
                        r.tasks + lv.first, lv.cnt_t, L, RING, g, r.tq);
-    hipLaunchKernelGGL(kern, dim3(std::min(units, C.ncu)), dim3(TILE_THREADS), 0, st, r.tasks + lv.first, L, RING, g,
+    const int per_cu = TILE_ONE(dpad) ? 2 : 1;
+    hipLaunchKernelGGL(kern, dim3(std::min(units, per_cu * C.ncu)), dim3(TILE_THREADS(dpad)), 0, st, r.tasks + lv.first, L, RING, g,
                        r.tq);
     HIPC(hipGetLastError());
     timed_end(tl);

@@ -1492,8 +1492,12 @@ __global__ __launch_bounds__(LEVEL_WG) void k_thin2(const LevelTask* __restrict_
 // L-1's plus the gains of the tiles' rows up to level L+i.
 #define TILE_RW 64                                // region side: tile + 2 * halo = one wave
 #define TILE_SLOTS (TILE_RW * TILE_RW)
-#define TILE_THREADS 1024
-#define TILE_PER_THREAD (TILE_SLOTS / TILE_THREADS)
+// threads of a k_tile workgroup: tables of at most 8 ids keep one copy of the
+// region (64 KiB, the next values in registers until a level is read) and two
+// workgroups of 512 a CU; wider ones two copies and one workgroup of 1024, since
+// their cells' offsets leave no registers for the next values
+#define TILE_ONE(DP) ((DP) <= 8)
+#define TILE_THREADS(DP) (TILE_ONE(DP) ? 512 : 1024)
 #define TILE_KMAX 8
 #define TILE_DPMAX 16                             // widest table k_tile takes
 
@@ -1582,22 +1586,29 @@ __global__ void k_tile_plan(const LevelTask* __restrict__ tasks, int ntasks, int
     const unsigned char* fr = T.chg0 + (g.fpar ^ 1) * 2 * ntiles;
     unsigned char* fw = T.chg0 + g.fpar * 2 * ntiles;
     const int tx = tile / g.tiles_y, ty = tile - tx * g.tiles_y;
-    bool active = g.first != 0 || fr[tile] != 0;
-    for (int ax = max(tx - 1, 0); ax <= min(tx + 1, g.tiles_x - 1) && !active; ax++)
-      for (int ay = max(ty - 1, 0); ay <= min(ty + 1, g.tiles_y - 1) && !active; ay++)
-        active = fr[ntiles + ax * g.tiles_y + ay] != 0;
+    // the tile and the 8 around it, read together (past the edge: the nearest)
+    u32 any = (u32)g.first | fr[tile];
+#pragma unroll
+    for (int d = 0; d < 9; d++) {
+      const int ax = min(max(tx + d / 3 - 1, 0), g.tiles_x - 1), ay = min(max(ty + d % 3 - 1, 0), g.tiles_y - 1);
+      any |= fr[ntiles + ax * g.tiles_y + ay];
+    }
+    const bool active = any != 0;
     if (active) tq[3 + atomicAdd(&tq[g.fpar], 1u)] = (u32)u;
     else { fw[tile] = 0; fw[ntiles + tile] = 0; }
   }
 }
 
-// k_tile: persistent workgroups (one per CU: the two region copies take
-// 128 KiB of LDS) pull units from the list until it is drained.  While a unit
-// runs its levels, the workgroup already claims the next unit and looks up its
-// cells' rows (after levels 0 and 1), so most of the chain of dependent global
-// loads a unit starts with overlaps the previous unit's levels.
+// k_tile: persistent workgroups pull units from the list until it is drained.
+// While a unit runs its levels, the workgroup already claims the next unit and
+// looks up its cells' rows (after levels 0 and 1), so most of the chain of
+// dependent global loads a unit starts with overlaps the previous unit's levels.
+// Bound by LDS reads (10.8 cycles a 16-byte neighbour read of a wave, conflicts
+// included); with two region copies and one workgroup a CU, nothing ran while a
+// unit was loaded, written back or waited at a barrier, 16 us a unit against the
+// 8 its reads take.  256 x 256 grid, d = 8: 144 -> 122 us a launch.
 
-// cell (lx, ly) of the region of a tile: thread tid owns (wave + 16 m, lane),
+// cell (lx, ly) of the region of a tile: thread tid owns (wave + waves m, lane),
 // a wave whole region columns
 struct TileUnit {
   int t, tile, tx, ty;
@@ -1609,11 +1620,13 @@ struct TileUnit {
 };
 
 template <int DP>
-__global__ __launch_bounds__(TILE_THREADS) void k_tile(const LevelTask* __restrict__ tasks, int level, int ring,
-                                                       TileArgs g, u32* __restrict__ tq)
+__global__ __launch_bounds__(TILE_THREADS(DP), 4) void k_tile(const LevelTask* __restrict__ tasks, int level, int ring,
+                                                              TileArgs g, u32* __restrict__ tq)
 {
-  __shared__ u64x2 rows[2][TILE_SLOTS];             // the region's chunks, cell (lx, ly) at lx * TILE_RW + ly
-  __shared__ u64 red[TILE_THREADS / 64][TILE_KMAX]; // per wave and level: gains of the tile's rows
+  constexpr bool ONE = TILE_ONE(DP);
+  constexpr int NW = TILE_THREADS(DP) / 64, PER = TILE_SLOTS / TILE_THREADS(DP);
+  __shared__ u64x2 rows[ONE ? 1 : 2][TILE_SLOTS];   // the region's chunks, cell (lx, ly) at lx * TILE_RW + ly
+  __shared__ u64 red[NW][TILE_KMAX];                // per wave and level: gains of the tile's rows
   __shared__ u32 claim_s;
   const int ntiles = g.tiles_x * g.tiles_y;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1621,8 +1634,8 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile(const LevelTask* __restri
   // rows of the unit's cells (-1: outside the grid) and their chunks
   auto cell_rows = [&](const TileUnit& U, int* rr) {
 #pragma unroll
-    for (int m = 0; m < TILE_PER_THREAD; m++) {
-      const int x = U.tx * g.tile - g.halo + wave + m * (TILE_THREADS / 64), y = U.ty * g.tile - g.halo + lane;
+    for (int m = 0; m < PER; m++) {
+      const int x = U.tx * g.tile - g.halo + wave + m * NW, y = U.ty * g.tile - g.halo + lane;
       rr[m] = (x >= 0 && x < g.width && y >= 0 && y < g.height) ? g.xy2row[x * g.height + y] : -1;
     }
   };
@@ -1630,7 +1643,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile(const LevelTask* __restri
     const LevelTask& T = tasks[U.t];
     const u64* __restrict__ in = g.dpar ? T.buf1 : T.buf0;
 #pragma unroll
-    for (int m = 0; m < TILE_PER_THREAD; m++) {
+    for (int m = 0; m < PER; m++) {
       vv[m].x = 0; vv[m].y = 0;
       if (rr[m] >= 0) vv[m] = *(const u64x2*)(in + (int64_t)rr[m] * T.kwp);
     }
@@ -1640,7 +1653,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile(const LevelTask* __restri
   const u32 q0 = __builtin_amdgcn_readfirstlane(claim_s);
   if (q0 >= nunits) return;                          // uniform
   u32 u = tq[3 + q0];
-  int rid[TILE_PER_THREAD];
+  int rid[PER];
   cell_rows(TileUnit(u, ntiles, g.tiles_y), rid);
   for (;;) {
     u32 claim = 0;
@@ -1651,38 +1664,37 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile(const LevelTask* __restri
     unsigned char* fw = T.chg0 + g.fpar * 2 * ntiles;
     u64* __restrict__ out = g.dpar ? T.buf0 : T.buf1;
     const int64_t kwp = T.kwp;
-    u32 off[TILE_PER_THREAD][DP / 2];
+    u32 off[ONE ? 2 : PER][DP / 2];                  // the cells' offsets (one copy: read again each level, a cell ahead)
     const u64 f0 = full_word(T.l, 0), f1 = full_word(T.l, 1);   // a saturated chunk
     bool nzv = false, usv = false;                   // some cell of the thread's is nonzero / unsaturated
     {
-      u64x2 val[TILE_PER_THREAD];
+      u64x2 val[PER];
       cell_chunks(U, rid, val);
 #pragma unroll
-      for (int m = 0; m < TILE_PER_THREAD; m++) {
-        rows[0][(wave + m * (TILE_THREADS / 64)) * TILE_RW + lane] = val[m];
+      for (int m = 0; m < PER; m++) {
+        rows[0][(wave + m * NW) * TILE_RW + lane] = val[m];
         nzv = nzv || (val[m].x | val[m].y) != 0;
         usv = usv || (rid[m] >= 0 && !(val[m].x == f0 && val[m].y == f1));
       }
     }
+    auto offsets = [&](int m, u32* w) {
+      // (a cell outside the grid reads row 0's: it is never updated)
+      const uint2* o = (const uint2*)(g.toff + (int64_t)max(rid[m], 0) * DP);
 #pragma unroll
-    for (int m = 0; m < TILE_PER_THREAD; m++) {
+      for (int j = 0; j < DP / 4; j++) { const uint2 v = o[j]; w[2 * j] = v.x; w[2 * j + 1] = v.y; }
+    };
+    if (!ONE)
 #pragma unroll
-      for (int j = 0; j < DP / 2; j++) off[m][j] = 0;
-      if (rid[m] >= 0) {
-        const uint2* o = (const uint2*)(g.toff + (int64_t)rid[m] * DP);
-#pragma unroll
-        for (int j = 0; j < DP / 4; j++) { const uint2 w = o[j]; off[m][2 * j] = w.x; off[m][2 * j + 1] = w.y; }
-      }
-    }
+      for (int m = 0; m < PER; m++) offsets(m, off[ONE ? 0 : m]);
     // a region whose cells are all zero, or all saturated, stays so for the k
     // levels: its tile is written back as loaded without running them (most
     // units of a first launch, and tiles the BFS front has just left)
     const bool any_nz = __syncthreads_or(nzv) != 0;
     const bool live = any_nz && __syncthreads_or(usv) != 0;
     u32 qn = nunits, un = 0;
-    int nrid[TILE_PER_THREAD];
+    int nrid[PER];
 #pragma unroll
-    for (int m = 0; m < TILE_PER_THREAD; m++) nrid[m] = -1;
+    for (int m = 0; m < PER; m++) nrid[m] = -1;
     if (!live) {
       if (tid == 0) claim_s = claim;
       __syncthreads();
@@ -1690,34 +1702,49 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile(const LevelTask* __restri
       if (qn < nunits) un = tq[3 + qn];
     }
     for (int i = 0; i < (live ? g.k : 0); i++) {
-      // level i reads copy i & 1 (level i - 1) and writes the other; cells it
-      // leaves out are never read again
-      const u64x2* __restrict__ src = rows[i & 1];
-      u64x2* __restrict__ dst = rows[(i + 1) & 1];
+      // level i reads copy i & 1 (level i - 1) and writes the other, or (one
+      // copy) writes it once every wave has read it; cells it leaves out are
+      // never read again
+      const u64x2* src = rows[ONE ? 0 : i & 1];
+      u64x2* dst = rows[ONE ? 0 : (i + 1) & 1];
+      u64x2 nx[ONE ? PER : 1];
       const int lo = (i + 1) * g.lmax, hi = TILE_RW - lo;
-      u32 gain = 0;                                  // at most 4 * 128 bits a thread
+      u32 gain = 0;                                  // at most 8 * 128 bits a thread
+      if (ONE) offsets(0, off[0]);
 #pragma unroll
-      for (int m = 0; m < TILE_PER_THREAD; m++) {
-        const int lx = wave + m * (TILE_THREADS / 64), sl = lx * TILE_RW + lane;
+      for (int m = 0; m < PER; m++) {
+        if (ONE && m + 1 < PER) offsets(m + 1, off[ONE ? (m + 1) & 1 : 0]);
+        const int lx = wave + m * NW, sl = lx * TILE_RW + lane;
         if (rid[m] >= 0 && lx >= lo && lx < hi && lane >= lo && lane < hi) {
           const u64x2 o = src[sl];
           u64x2 x = o;
           // a saturated chunk gains nothing: its neighbours are not read
-          if (!(o.x == f0 && o.y == f1))
+          if (!(o.x == f0 && o.y == f1)) {
+            const u32* w = off[ONE ? m & 1 : m];
 #pragma unroll
           for (int j = 0; j < DP / 2; j++) {
             // the window keeps every neighbour inside the region: a cell at least
             // (i + 1) lmax from its edges, and no offset longer than lmax cells
             // (k_tgeom flags longer ones, which end the run)
-            const int s0 = sl + (int)(short)(off[m][j] & 0xffff);
-            const int s1 = sl + (int)(short)(off[m][j] >> 16);
+            const int s0 = sl + (int)(short)(w[j] & 0xffff);
+            const int s1 = sl + (int)(short)(w[j] >> 16);
             const u64x2 a = src[s0], c = src[s1];
             x.x |= a.x | c.x;
             x.y |= a.y | c.y;
           }
-          dst[sl] = x;
+          }
+          if (ONE) nx[ONE ? m : 0] = x;
+          else dst[sl] = x;
           if (lx >= g.halo && lx < g.halo + g.tile && lane >= g.halo && lane < g.halo + g.tile)
             gain += (u32)(__popcll(x.x ^ o.x) + __popcll(x.y ^ o.y));   // x holds o: its new bits
+        }
+      }
+      if (ONE) {
+        __syncthreads();                             // level i - 1 is read
+#pragma unroll
+        for (int m = 0; m < PER; m++) {
+          const int lx = wave + m * NW;
+          if (rid[m] >= 0 && lx >= lo && lx < hi && lane >= lo && lane < hi) dst[lx * TILE_RW + lane] = nx[ONE ? m : 0];
         }
       }
       const u64 wgain = wave_sum((u64)gain);
@@ -1735,15 +1762,15 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile(const LevelTask* __restri
     if ((!live || g.k < 2) && qn < nunits) cell_rows(TileUnit(un, ntiles, g.tiles_y), nrid);   // not yet
     // the tile's rows, its counts and flags
 #pragma unroll
-    for (int m = 0; m < TILE_PER_THREAD; m++) {
-      const int lx = wave + m * (TILE_THREADS / 64);
+    for (int m = 0; m < PER; m++) {
+      const int lx = wave + m * NW;
       if (rid[m] >= 0 && lx >= g.halo && lx < g.halo + g.tile && lane >= g.halo && lane < g.halo + g.tile)
-        *(u64x2*)(out + (int64_t)rid[m] * kwp) = rows[live ? (g.k & 1) : 0][lx * TILE_RW + lane];
+        *(u64x2*)(out + (int64_t)rid[m] * kwp) = rows[live && !ONE ? (g.k & 1) : 0][lx * TILE_RW + lane];
     }
     if (tid < g.k) {
       u64 cum = 0, last = 0;
       for (int i = 0; live && i <= tid; i++)
-        for (int w = 0; w < TILE_THREADS / 64; w++) { cum += red[w][i]; if (i == tid) last += red[w][i]; }
+        for (int w = 0; w < NW; w++) { cum += red[w][i]; if (i == tid) last += red[w][i]; }
       if (cum) atomicAdd(&T.cnt[(int64_t)((level + tid) % ring) * cs], cum);
       if (tid == g.k - 1) {
         fw[U.tile] = cum != 0;
@@ -1756,7 +1783,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile(const LevelTask* __restri
     if (qn >= nunits) break;                         // uniform
     u = un;
 #pragma unroll
-    for (int m = 0; m < TILE_PER_THREAD; m++) rid[m] = nrid[m];
+    for (int m = 0; m < PER; m++) rid[m] = nrid[m];
   }
 }
 
