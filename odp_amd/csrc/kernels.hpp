@@ -1554,6 +1554,24 @@ __global__ void k_tgeom(const int* __restrict__ nbr, int n, int dpad, const int*
   }
 }
 
+// the longest |dx| or |dy| of an adjacency entry (ids outside the grid skipped),
+// into *lmax (zero before the launch).  Row i is base vertex i, or (s = 4) the
+// i-th vertex of the first quadrant.  Bound by the waves' adds to one word: eight
+// entries a thread and a look at the word first (131072 entries: 25.6 -> 7.4 us).
+__global__ void k_lmax(const int* __restrict__ adj, int rows, int degree, int width, int height, int s, int* lmax)
+{
+  const int bh = height / 2, n = width * height;
+  int m = 0;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < rows * degree; i += gridDim.x * blockDim.x) {
+    const int r = i / degree, u = adj[i];
+    const int v = s == 4 ? (r / bh) * height + (r % bh) : r;
+    if (u >= 0 && u < n) m = max(m, max(abs(u / height - v / height), abs(u % height - v % height)));
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
+  if ((threadIdx.x & 63) == 0 && m > __hip_atomic_load(lmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(lmax, m);
+}
+
 // k_tile_plan: per (task, tile) unit of the launch: k_level's stop test, the
 // count slots of levels L..L+k-1 (tile 0 of a task), and the activity test;
 // the active units go to a list that k_tile's workgroups drain.
