@@ -2042,8 +2042,18 @@ __global__ __launch_bounds__(1024) void k_direct(DirectArgs a)
 // tid, tid+nth, ... (at most RPT of them) and keeps their next values in
 // registers until the whole workgroup has read the level, then writes them
 // back, so one buffer of n*WB*4 bytes suffices (two barriers per level).
-// Neighbour ids are read as 16-bit row indices (graphs here have n <= 32768),
-// eight per 16-byte load.
+// Neighbour ids are read as 16-bit row indices, eight per 16-byte load.
+// The pulled levels of a large block are bound by LDS reads of random rows: 9 to
+// 9.5 cycles a wave's read of 4 or 8 bytes a lane, bank conflicts included (n =
+// 30002, d = 7: 34k cycles a level of 3750 reads), so the block is as wide as
+// LDS allows.  Small blocks are bound by the chain from one level to the next;
+// what lay on it besides the reads: the own row's read and the wait for its ids
+// (kept in registers, and fetched a row ahead, across the barrier too), the
+// count's trips through LDS shuffles (now adds between lanes, 32 bits), and the
+// passes over empty rows of the unrolled loops (now left at the last row).  A
+// pulled level of n = 1024, d = 6 takes 2300 cycles of 6000 before; one
+// evaluation n = 1024 26.8 -> 24.0 us, n = 5001, d = 10 49.2 -> 41.0,
+// n = 30002, d = 7 375 -> 342.
 
 struct ResTask {
   const unsigned short* nbr;   // [n][dp] 16-bit row indices, padded with the row itself
@@ -2093,9 +2103,8 @@ struct ResOut {     // per-graph accumulators
 __host__ __device__ constexpr int res_rpt(int wb) { return wb == 1 ? 16 : wb == 2 ? 16 : wb == 4 ? 10 : 2; }
 // rows per thread of the single-graph instances past 16384 rows, for two-word
 // blocks (their LDS buffer holds up to 20416 rows) and one-word blocks (up to
-// 40832 rows: 28 rows a thread without spills, 32 and 40 with 52 and 196 bytes
-// a lane spilled, still as fast as the level plan or faster at every degree):
-// instantiations of their own, so that the other launches keep their registers
+// 40832 rows; 62 to 74 registers): instantiations of their own, so that the
+// other launches keep their registers
 #define RES_RPT_WIDE 20
 #define RES_RPT_WIDE1 28
 #define RES_RPT_WIDE1B 32
@@ -2205,25 +2214,66 @@ __device__ __forceinline__ u64 uniform_u64(u64 v)
   return ((u64)hi << 32) | lo;
 }
 
-__device__ __forceinline__ u64 block_total(u64 v, u64* part, int wave, int nw)
+// the wave's sum, by adds between lanes (DPP: no LDS trips, as shuffles make);
+// the same value in every lane, in a scalar register
+__device__ __forceinline__ u32 wave_sum_dpp(u32 v)
 {
-  v = wave_sum(v);      // every lane holds the wave total: all write the same value
-  part[wave] = v;
-  __syncthreads();
-  u64 s = 0;
-  for (int i = 0; i < nw; i++) s += part[i];
-  return uniform_u64(s);
+  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);   // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);   // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);   // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);   // row_bcast:15
+  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);   // row_bcast:31
+  return (u32)__builtin_amdgcn_readlane((int)v, 63);
 }
+
+// part: 16 words a wave each, those past the workgroup's waves zero
+__device__ __forceinline__ u32 block_total(u32 v, u32* part, int wave)
+{
+  part[wave] = wave_sum_dpp(v);      // every lane writes the same value
+  __syncthreads();
+  u32 s = 0;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const uint4 q = ((const uint4*)part)[i];
+    s += q.x + q.y + q.z + q.w;
+  }
+  return (u32)__builtin_amdgcn_readfirstlane((int)s);
+}
+
+// v again, as far as the compiler can tell a new value: what is computed from
+// it is not kept in registers across the loop around it
+__device__ __forceinline__ int again(int v)
+{
+  asm volatile("" : "+s"(v));
+  return v;
+}
+
+// Division of numbers below 2^24 by one divisor: the float quotient is at most
+// one off.
+struct FastDiv {
+  u32 d;
+  float inv;
+  __device__ __forceinline__ explicit FastDiv(u32 v) : d(v), inv(1.0f / (float)v) {}
+  __device__ __forceinline__ u32 div(u32 x, u32& rem) const
+  {
+    u32 q = (u32)((float)x * inv);
+    int r = (int)(x - q * d);
+    if (r < 0) { q--; r += (int)d; }
+    else if (r >= (int)d) { q++; r -= (int)d; }
+    rem = (u32)r;
+    return q;
+  }
+};
 
 // All levels of one block of T.l <= 32*WB sources; returns the block's totals
 // (the same value in every thread).
-// MAD: pulled rows address their neighbours with row_or2 (k_anneal keeps
-// row_or: its larger register set spills more with it)
-template <int WB, bool STOP = false, bool WALK = true, bool MAD = true, int RPT = res_rpt(WB)>
-__device__ __forceinline__ ResOut res_run(const ResTask& T, u32* cur, u64 (*s_part)[16],
-                                          int tid, int nth, int lane, int wave, int nw)
+// The counts fit 32 bits: a block is at most 160 KiB of them.
+template <int WB, bool STOP = false, bool WALK = true, int RPT = res_rpt(WB)>
+__device__ __forceinline__ ResOut res_run(const ResTask& T, u32* cur, u32 (*s_part)[16],
+                                          int tid, int nth, int wave)
 {
-  const u64 target = (u64)T.n * (u64)T.l;
+  const u32 target = (u32)T.n * (u32)T.l;
   const u32 cbase = (u32)(uintptr_t)(__attribute__((address_space(3))) u32*)cur;   // cur's LDS byte address
   RowT<WB> full;
 #pragma unroll
@@ -2232,29 +2282,23 @@ __device__ __forceinline__ ResOut res_run(const ResTask& T, u32* cur, u64 (*s_pa
     full.w[k] = v >= 32 ? ~0u : (v <= 0 ? 0u : ((1u << v) - 1u));
   }
   // level 0 straight from the identity: row r holds r and its neighbours
-  u64 pop = 0;
+  u32 pop = 0;
   if (WALK && T.walk >= 1) {
     // from the sources' side: clear every row, then each source sets its bit
-    // in its own row and in its neighbours' rows (the table is symmetric)
-    for (int r = tid; r < T.n; r += nth) {
-      RowT<WB> row;
-#pragma unroll
-      for (int k = 0; k < WB; k++) row.w[k] = 0;
-      lds_store<WB>(cur + r * WB, row);
-    }
+    // in its own row and in its neighbours' rows (the table is symmetric);
+    // whoever finds a bit clear counts it
+    const int words = T.n * WB;
+    for (int w = 4 * tid; w < (words & ~3); w += 4 * nth) *(uint4*)(cur + w) = make_uint4(0, 0, 0, 0);
+    if (tid < (words & 3)) cur[(words & ~3) + tid] = 0;
     __syncthreads();
-    const int per = T.deg + 1;
-    for (int it = tid; it < T.l * per; it += nth) {
-      const int c0 = it / per, j = it - c0 * per;
-      const int src = T.src0 + c0;
-      const int v = j == T.deg ? src : (int)T.nbr[src * T.dp + j];
-      atomicOr(&cur[v * WB + (c0 >> 5)], 1u << (c0 & 31));
-    }
-    __syncthreads();
-    for (int r = tid; r < T.n; r += nth) {
-      const RowT<WB> row = lds_row<WB>(cur + r * WB);
-#pragma unroll
-      for (int k = 0; k < WB; k++) pop += (u64)__popc(row.w[k]);
+    const FastDiv per((u32)T.deg + 1);
+    for (u32 it = (u32)tid; it < (u32)T.l * per.d; it += (u32)nth) {
+      u32 j;
+      const u32 c0 = per.div(it, j);
+      const int src = T.src0 + (int)c0;
+      const int v = j == (u32)T.deg ? src : (int)T.nbr[src * T.dp + (int)j];
+      const u32 b = 1u << (c0 & 31);
+      pop += (atomicOr(&cur[v * WB + (int)(c0 >> 5)], b) & b) == 0;
     }
   } else
   for (int r = tid; r < T.n; r += nth) {
@@ -2280,121 +2324,132 @@ __device__ __forceinline__ ResOut res_run(const ResTask& T, u32* cur, u64 (*s_pa
     }
     lds_store<WB>(cur + r * WB, row);
 #pragma unroll
-    for (int k = 0; k < WB; k++) pop += (u64)__popc(row.w[k]);
+    for (int k = 0; k < WB; k++) pop += (u32)__popc(row.w[k]);
   }
   int par = 0;
-  u64 c = block_total(pop, s_part[par], wave, nw);
-  u64 prev = 0, sum = 0;
+  u32 c = block_total(pop, s_part[par], wave);
+  u32 prev = 0;
+  u64 sum = 0;
   int L = 0, D = 0;
   bool disc = false;
+  // (n = 30002, d = 7: level 0 8.4k -> 3.2k cycles, the walked third 11.5k -> 5.7k,
+  // with the counts taken from the bit-sets instead of a pass over the rows)
   // levels 1 .. T.walk - 1: the walks of exactly L + 1 steps from each source
   // set its bit in the rows they end at (the rows already hold level L - 1,
   // every shorter walk); the exits are left to the pulled levels' loop below
   while (WALK && L + 1 < T.walk && c != target && !(L >= 1 && c == prev) && L + 1 < T.n) {
-    sum += (target - c) * (u64)T.s;
+    sum += (u64)(target - c) * (u64)T.s;
     prev = c;
     L++;
-    const u32 deg = (u32)T.deg, steps = (u32)L + 1;
+    const u32 steps = (u32)L + 1;
     // a thread takes a walk's first steps - 1 steps (its prefix, decoded with
     // divisions) and then every last step at once: the whole table row of the
     // vertex reached, 8 ids a load -- deg walks per decoded prefix
-    u32 per = 1;
-    for (u32 i = 0; i + 1 < steps; i++) per *= deg;
-    const u32 prefixes = (u32)T.l * per;
-    for (u32 it = (u32)tid; it < prefixes; it += (u32)nth) {
-      const u32 c0 = it / per;
-      u32 rem = it - c0 * per;
+    u32 all = 1;
+    for (u32 i = 0; i + 1 < steps; i++) all *= (u32)T.deg;
+    const FastDiv per(all), deg((u32)T.deg);
+    pop = 0;
+    for (u32 it = (u32)tid; it < (u32)T.l * all; it += (u32)nth) {
+      u32 rem;
+      const u32 c0 = per.div(it, rem);
       int v = T.src0 + (int)c0;
       for (u32 i = 0; i + 1 < steps; i++) {
-        const u32 j = rem % deg;
-        rem /= deg;
+        u32 j;
+        rem = deg.div(rem, j);
         v = T.nbr[v * T.dp + (int)j];
       }
       u32* col = cur + (int)(c0 >> 5);
       const u32 b = 1u << (c0 & 31);
+      auto set2 = [&](u32 g) {
+        const u32 x = atomicOr(col + (g & 0xffff) * WB, b), y = atomicOr(col + (g >> 16) * WB, b);
+        pop += ((x & b) == 0) + ((y & b) == 0);
+      };
       const uint4* ids = (const uint4*)(T.nbr + v * T.dp);
       for (int q = 0; q < (T.dq >> 1); q++) {
         const uint4 g = ids[q];
-        atomicOr(col + (g.x & 0xffff) * WB, b); atomicOr(col + (g.x >> 16) * WB, b);
-        atomicOr(col + (g.y & 0xffff) * WB, b); atomicOr(col + (g.y >> 16) * WB, b);
-        atomicOr(col + (g.z & 0xffff) * WB, b); atomicOr(col + (g.z >> 16) * WB, b);
-        atomicOr(col + (g.w & 0xffff) * WB, b); atomicOr(col + (g.w >> 16) * WB, b);
+        set2(g.x); set2(g.y); set2(g.z); set2(g.w);
       }
       if (T.dq & 1) {
         const uint2 g = ((const uint2*)ids)[T.dq - 1];
-        atomicOr(col + (g.x & 0xffff) * WB, b); atomicOr(col + (g.x >> 16) * WB, b);
-        atomicOr(col + (g.y & 0xffff) * WB, b); atomicOr(col + (g.y >> 16) * WB, b);
+        set2(g.x); set2(g.y);
       }
     }
-    __syncthreads();
-    pop = 0;
-    for (int r = tid; r < T.n; r += nth) {
-      const RowT<WB> row = lds_row<WB>(cur + r * WB);
-#pragma unroll
-      for (int k = 0; k < WB; k++) pop += (u64)__popc(row.w[k]);
-    }
     par ^= 1;
-    c = block_total(pop, s_part[par], wave, nw);
+    c += block_total(pop, s_part[par], wave);
+  }
+  // the pulled levels: a thread's own rows stay in registers from level to level
+  RowT<WB> own[RPT];
+  uint4 w0 = make_uint4(0, 0, 0, 0), w1 = w0;      // the first 16 ids of the row fetched last
+  bool live = false;                               // ... which has bits to gain
+  auto is_full = [&](const RowT<WB>& q) {
+    bool f = true;
+#pragma unroll
+    for (int k = 0; k < WB; k++) f = f && q.w[k] == full.w[k];
+    return f;
+  };
+  auto ids_at = [&](int i, int nl) { return (const uint4*)(T.nbr + (int64_t)(i * nl) * T.dp) + (u32)tid * (u32)(T.dp >> 3); };
+  auto fetch = [&](int i, int nl) {
+    live = tid + i * nl < T.n && !is_full(own[i]);
+    if (live) {
+      const uint4* ids = ids_at(i, nl);
+      w0 = ids[0];
+      if (T.dq > 2) w1 = ids[1];
+    }
+  };
+  if (c != target) {
+    const int nl = again(nth);
+#pragma unroll
+    for (int i = 0; i < RPT; i++) {
+      const int r = tid + i * nl;
+      if (r < T.n) own[i] = lds_row<WB>(cur + r * WB);
+      else
+#pragma unroll
+        for (int k = 0; k < WB; k++) own[i].w[k] = 0;
+    }
+    fetch(0, nl);
   }
   for (;;) {
     if (c == target) { D = L + 1; break; }
     if ((L >= 1 && c == prev) || L + 1 >= T.n) { disc = true; break; }
-    sum += (target - c) * (u64)T.s;
+    sum += (u64)(target - c) * (u64)T.s;
     prev = c;
     L++;
-    RowT<WB> nx[RPT];
     pop = 0;
+    const int nl = again(nth);
 #pragma unroll
     for (int i = 0; i < RPT; i++) {
-      const int r = tid + i * nth;
-      if (r < T.n) {
-        RowT<WB> row = lds_row<WB>(cur + r * WB);
-        bool sat = true;
-#pragma unroll
-        for (int k = 0; k < WB; k++) sat = sat && (row.w[k] == full.w[k]);
-        if (!sat) {
-          const uint4* ids = (const uint4*)T.nbr;
-          const u32 off = (u32)r * (u32)(T.dp >> 3);
-          bool done = false;
-          for (int j = 0; j < (T.dq >> 1); j++) {
-            const uint4 v = ids[off + j];
-            if (MAD) {
-              row_or2<WB>(row, cbase, v.x); row_or2<WB>(row, cbase, v.y);
-              row_or2<WB>(row, cbase, v.z); row_or2<WB>(row, cbase, v.w);
-            } else {
-              row_or<WB>(row, cur, v.x & 0xffff); row_or<WB>(row, cur, v.x >> 16);
-              row_or<WB>(row, cur, v.y & 0xffff); row_or<WB>(row, cur, v.y >> 16);
-              row_or<WB>(row, cur, v.z & 0xffff); row_or<WB>(row, cur, v.z >> 16);
-              row_or<WB>(row, cur, v.w & 0xffff); row_or<WB>(row, cur, v.w >> 16);
-            }
-            if (STOP) {                            // a row filled by 8 neighbours reads no more
-              done = true;
-#pragma unroll
-              for (int k = 0; k < WB; k++) done = done && (row.w[k] == full.w[k]);
-              if (done) break;
-            }
-          }
-          if ((T.dq & 1) && !done) {
-            const uint2 v = ((const uint2*)T.nbr)[2 * off + (T.dq - 1)];
-            if (MAD) {
-              row_or2<WB>(row, cbase, v.x); row_or2<WB>(row, cbase, v.y);
-            } else {
-              row_or<WB>(row, cur, v.x & 0xffff); row_or<WB>(row, cur, v.x >> 16);
-              row_or<WB>(row, cur, v.y & 0xffff); row_or<WB>(row, cur, v.y >> 16);
-            }
+      if (i > 0 && i * nl >= T.n) break;           // uniform
+      // the next row's ids are on their way while this row's neighbours are read
+      const uint4 v0 = w0, v1 = w1;
+      const bool need = live;
+      live = false;
+      if (i + 1 < RPT) fetch(i + 1, nl);
+      if (need) {
+        row_or2<WB>(own[i], cbase, v0.x); row_or2<WB>(own[i], cbase, v0.y);
+        if (T.dq > 1) { row_or2<WB>(own[i], cbase, v0.z); row_or2<WB>(own[i], cbase, v0.w); }
+        if (T.dq > 2 && !(STOP && is_full(own[i]))) {        // STOP: a row filled by 8 neighbours reads no more
+          row_or2<WB>(own[i], cbase, v1.x); row_or2<WB>(own[i], cbase, v1.y);
+          if (T.dq > 3) { row_or2<WB>(own[i], cbase, v1.z); row_or2<WB>(own[i], cbase, v1.w); }
+          for (int j = 4; j < T.dq && !(STOP && is_full(own[i])); j++) {
+            const uint2 v = ((const uint2*)ids_at(i, nl))[j];
+            row_or2<WB>(own[i], cbase, v.x); row_or2<WB>(own[i], cbase, v.y);
           }
         }
-        nx[i] = row;
-#pragma unroll
-        for (int k = 0; k < WB; k++) pop += (u64)__popc(row.w[k]);
       }
-    }
-    par ^= 1;
-    c = block_total(pop, s_part[par], wave, nw);   // every read of this level is done
 #pragma unroll
-    for (int i = 0; i < RPT; i++) {
-      const int r = tid + i * nth;
-      if (r < T.n) lds_store<WB>(cur + r * WB, nx[i]);
+      for (int k = 0; k < WB; k++) pop += (u32)__popc(own[i].w[k]);
+    }
+    fetch(0, nl);                                // the next level's first row, ahead of the barriers
+    par ^= 1;
+    c = block_total(pop, s_part[par], wave);   // every read of this level is done
+    {
+      const int nl = again(nth);
+#pragma unroll
+      for (int i = 0; i < RPT; i++) {
+        if (i > 0 && i * nl >= T.n) break;
+        const int r = tid + i * nl;
+        if (r < T.n) lds_store<WB>(cur + r * WB, own[i]);
+      }
     }
     __syncthreads();                               // the new level is visible
   }
@@ -2550,9 +2605,10 @@ __global__ __launch_bounds__(1024) void k_resident_w(const ResTask* __restrict__
 {
   extern __shared__ __attribute__((aligned(16))) u32 lds[];
   __shared__ int s_task, s_last;
-  __shared__ u64 s_part[2][16];
+  __shared__ __attribute__((aligned(16))) u32 s_part[2][16];
   const int tid = threadIdx.x, nth = blockDim.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = nth >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (tid < 32 && (tid & 15) >= (nth + 63) / 64) s_part[tid >> 4][tid & 15] = 0;
   ResOut mine;           // this workgroup's totals (single-graph launches)
   mine.sum = 0; mine.diam = 0; mine.flags = 0; mine.levels = 0; mine.pad = 0;
   if (fin.patch.n) {     // uniform: a kernel argument
@@ -2566,11 +2622,12 @@ __global__ __launch_bounds__(1024) void k_resident_w(const ResTask* __restrict__
   // from *qhead (which then counts past gridDim.x)
   int t = blockIdx.x;
   while (t < ntasks) {
-    const ResOut b = res_run<WB, STOP, true, true, RPT>(tasks[t], lds, s_part, tid, nth, lane, wave, nw);
+    const ResTask T = tasks[t];
+    const ResOut b = res_run<WB, STOP, true, RPT>(T, lds, s_part, tid, nth, wave);
     if (fin.done) {
       mine.sum += b.sum; mine.diam = max(mine.diam, b.diam); mine.flags |= b.flags; mine.levels += b.levels;
     } else {
-      res_commit(out, tasks[t].graph, b, lane, wave);
+      res_commit(out, T.graph, b, lane, wave);
     }
     if ((int)gridDim.x >= ntasks) break;          // nothing left to pop
     if (wave == 0) {       // wave-uniform: lane 0 adds 1, the others add 0
@@ -2601,9 +2658,10 @@ __global__ __launch_bounds__(1024) void k_resident(const ResTask* __restrict__ t
 {
   extern __shared__ __attribute__((aligned(16))) u32 lds[];
   __shared__ int s_task;
-  __shared__ u64 s_part[2][16];
+  __shared__ __attribute__((aligned(16))) u32 s_part[2][16];
   const int tid = threadIdx.x, nth = blockDim.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = nth >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (tid < 32 && (tid & 15) >= (nth + 63) / 64) s_part[tid >> 4][tid & 15] = 0;
   for (;;) {
     if (wave == 0) {       // wave-uniform: lane 0 adds 1, the others add 0
       const int got = atomicAdd(qhead, lane == 0 ? 1 : 0);
@@ -2615,10 +2673,10 @@ __global__ __launch_bounds__(1024) void k_resident(const ResTask* __restrict__ t
     const ResTask T = tasks[t];
     ResOut b;
     switch (T.wb) {
-      case 1: b = res_run<1>(T, lds, s_part, tid, nth, lane, wave, nw); break;
-      case 2: b = res_run<2>(T, lds, s_part, tid, nth, lane, wave, nw); break;
-      case 4: b = res_run<4>(T, lds, s_part, tid, nth, lane, wave, nw); break;
-      default: b = res_run<8>(T, lds, s_part, tid, nth, lane, wave, nw); break;
+      case 1: b = res_run<1>(T, lds, s_part, tid, nth, wave); break;
+      case 2: b = res_run<2>(T, lds, s_part, tid, nth, wave); break;
+      case 4: b = res_run<4>(T, lds, s_part, tid, nth, wave); break;
+      default: b = res_run<8>(T, lds, s_part, tid, nth, wave); break;
     }
     res_commit(out, T.graph, b, lane, wave);
   }
@@ -2700,13 +2758,14 @@ template <int WB>
 __global__ __launch_bounds__(1024) void k_anneal(AnnealArgs a)
 {
   extern __shared__ __attribute__((aligned(16))) u32 lds[];
-  __shared__ u64 s_part[2][16];
+  __shared__ __attribute__((aligned(16))) u32 s_part[2][16];
   __shared__ int s_mv[5], s_dec[3];
   __shared__ u64 s_sum;
   __shared__ int s_diam, s_flags;
   __shared__ AnnealState S;          // the chain's state; only thread 0 reads or writes it
   const int tid = threadIdx.x, nth = blockDim.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = nth >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (tid < 32 && (tid & 15) >= (nth + 63) / 64) s_part[tid >> 4][tid & 15] = 0;
   const int g = blockIdx.x, G = gridDim.x, n = a.n, deg = a.degree, dp = a.dp;
   u32* bits = lds;
   unsigned short* tab = (unsigned short*)(lds + ((n * WB + 3) & ~3));
@@ -2739,7 +2798,7 @@ __global__ __launch_bounds__(1024) void k_anneal(AnnealArgs a)
       if (tid == 0) S.stop = 1;
       break;
     }
-    const ResOut b = res_run<WB, false, false, false>(T, bits, s_part, tid, nth, lane, wave, nw);   // no walks (measured faster)
+    const ResOut b = res_run<WB, false, false>(T, bits, s_part, tid, nth, wave);   // no walks (measured faster)
     const int par = k & 1;                             // slots of this step (k is uniform; S.steps is thread 0's)
     if (tid == 0) {
       a.slots[par * G + g] = b;
