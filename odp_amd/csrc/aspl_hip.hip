@@ -2390,10 +2390,9 @@ static void anneal_on_device(Evaluator& v, int* adj_out, const std::vector<int>&
   S.cur_d = cur_d; S.best_d = best_d; S.low_d = low_d;
   S.hill = hill ? 1 : 0; S.prio = prio ? 1 : 0;
   AnnealState* d_st = nullptr;
-  ResOut* d_slots = nullptr;
-  u32* d_bar = nullptr;
+  u64* d_slots = nullptr;
   int* d_best = nullptr;
-  dalloc(&d_st, 1); dalloc(&d_slots, (size_t)2 * G); dalloc(&d_bar, 1); dalloc(&d_best, (size_t)n * deg);
+  dalloc(&d_st, 1); dalloc(&d_slots, (size_t)2 * G); dalloc(&d_best, (size_t)n * deg);
   HIPC(hipMemcpyAsync(d_st, &S, sizeof S, hipMemcpyHostToDevice, C.stream));
   const size_t lds = anneal_lds(v);
   const void* f = wb == 1 ? (const void*)k_anneal<1> : wb == 2 ? (const void*)k_anneal<2>
@@ -2402,10 +2401,10 @@ static void anneal_on_device(Evaluator& v, int* adj_out, const std::vector<int>&
   const double t_dev = wall_time();
   while (S.steps < ncalcs && !S.optimum && !S.stop) {
     AnnealArgs aa;
-    aa.adj = v.d_adj; aa.best = d_best; aa.st = d_st; aa.slots = d_slots; aa.bar = d_bar;
+    aa.adj = v.d_adj; aa.best = d_best; aa.st = d_st; aa.slots = d_slots;
     aa.n = n; aa.degree = deg; aa.dp = v.dp16; aa.ntasks = G;
     aa.steps = (int)std::min<long long>(chunk, ncalcs - S.steps);
-    hipLaunchKernelGGL(k_clear, dim3(1), dim3(64), 0, C.stream, (u64*)nullptr, 0, (int*)d_bar, 1);
+    hipLaunchKernelGGL(k_clear, dim3((2 * G + 63) / 64), dim3(64), 0, C.stream, d_slots, 2 * G, (int*)nullptr, 0);
     void* args[] = {&aa};
     HIPC(hipLaunchCooperativeKernel(f, dim3(G), dim3(v.rr.threads), args, (unsigned)lds, C.stream));
     HIPC(hipMemcpyAsync(&S, d_st, sizeof S, hipMemcpyDeviceToHost, C.stream));
@@ -2419,7 +2418,7 @@ static void anneal_on_device(Evaluator& v, int* adj_out, const std::vector<int>&
     HIPC(hipMemcpy(adj_out, d_best, sizeof(int) * (size_t)n * deg, hipMemcpyDeviceToHost));
   else
     memcpy(adj_out, start.data(), sizeof(int) * (size_t)n * deg);
-  dfree(&d_st); dfree(&d_slots); dfree(&d_bar); dfree(&d_best);
+  dfree(&d_st); dfree(&d_slots); dfree(&d_best);
   // the device copy now holds the chain's current graph; the 16-bit table is rebuilt from it
   v.stage_is_device = false;
   v.mirror_ok = false;

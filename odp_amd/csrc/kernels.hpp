@@ -2689,13 +2689,18 @@ __global__ __launch_bounds__(1024) void k_resident(const ResTask* __restrict__ t
 //
 // Every workgroup holds the whole 16-bit neighbour table in LDS (the first
 // `degree` entries of a row are its adjacency row) and evaluates one block of
-// 32 * WB sources.  Thread 0 of every workgroup keeps the same copy of the
+// 32 * WB sources.  Wave 0 of every workgroup keeps the same copy of the
 // chain's state -- generator, current and best results, temperature -- and
 // draws the same 2-opt move the host's ODPX_Two_opt would draw from it, so the
-// tables stay identical without any exchange.  One grid barrier per step: each
-// workgroup publishes its block's totals, waits for all of them, adds them up
-// in the same order and makes the same acceptance decision (the test of
+// tables stay identical without any exchange.  Each step every workgroup
+// publishes its block's totals in one word, watches for all the others', adds
+// them up in the same order and makes the same acceptance decision (the test of
 // sample/SA/common.c:15-43); a rejected move is undone in every table.
+// Bound by the chain of a step: move, levels, totals across the XCDs, decision.
+// One thread that searched the rows entry by entry, an arrival counter with a
+// second read of the totals after it, and six workgroup barriers took 12.6 us a
+// step at n = 1024, d = 6; rows searched by the wave's lanes, totals that carry
+// their own arrival and two barriers 10.5.
 
 struct AnnealState {
   uint64_t rng[4];
@@ -2712,8 +2717,7 @@ struct AnnealArgs {
   int* adj;             // [n][degree]: the chain's current graph (read at start, written at the end)
   int* best;            // [n][degree]: the best graph, written on every improvement
   AnnealState* st;
-  ResOut* slots;        // [2][ntasks] block totals of a step (double buffered by step parity)
-  u32* bar;             // grid barrier counter (zero at launch)
+  u64* slots;           // [2][ntasks] packed block totals of a step (by step parity; zero at launch)
   int n, degree, dp, ntasks, steps;
 };
 
@@ -2734,24 +2738,39 @@ __device__ __forceinline__ uint64_t anneal_next(uint64_t s[4])
   return r;
 }
 
-__device__ __forceinline__ bool anneal_has(const unsigned short* tab, int dp, int degree, int a, int b)
+// first position of id among a row's entries, -1 if none; the wave's lanes look
+// at 64 entries together, every lane returns the same value
+__device__ __forceinline__ int anneal_find(const unsigned short* tab, int dp, int degree, int row, int id, int lane)
 {
-  for (int j = 0; j < degree; j++) if (tab[a * dp + j] == b) return true;
-  return false;
+  for (int j = 0; j < degree; j += 64) {
+    const u64 hit = __ballot(j + lane < degree && tab[row * dp + j + lane] == id);
+    if (hit) return j + __ffsll((unsigned long long)hit) - 1;
+  }
+  return -1;
 }
 
-__device__ __forceinline__ void anneal_replace(unsigned short* tab, int dp, int degree, int row, int from, int to)
+__device__ __forceinline__ void anneal_replace(unsigned short* tab, int dp, int degree, int row, int from, int to, int lane)
 {
-  for (int j = 0; j < degree; j++) if (tab[row * dp + j] == from) { tab[row * dp + j] = (unsigned short)to; return; }
+  const int j = anneal_find(tab, dp, degree, row, from, lane);
+  if (j >= 0) tab[row * dp + j] = (unsigned short)to;
 }
 
-// a-b, c-d -> a-c, b-d in the table (ODPX_Swap_edges' order of replacements)
-__device__ __forceinline__ void anneal_swap(unsigned short* tab, int dp, int degree, int a, int b, int c, int d)
+// a-b, c-d -> a-c, b-d in the table (ODPX_Swap_edges' order of replacements), by one wave
+__device__ __forceinline__ void anneal_swap(unsigned short* tab, int dp, int degree, int a, int b, int c, int d, int lane)
 {
-  anneal_replace(tab, dp, degree, a, b, c);
-  anneal_replace(tab, dp, degree, b, a, d);
-  anneal_replace(tab, dp, degree, c, d, a);
-  anneal_replace(tab, dp, degree, d, c, b);
+  anneal_replace(tab, dp, degree, a, b, c, lane);
+  anneal_replace(tab, dp, degree, b, a, d, lane);
+  anneal_replace(tab, dp, degree, c, d, a, lane);
+  anneal_replace(tab, dp, degree, d, c, b, lane);
+}
+
+// A block's totals of one step in one word, so that a workgroup's slot is
+// complete whenever it is read: sum (bits 0..39: at most n levels of the 1.3 M
+// bits a block's LDS holds), diameter (40..53: n <= 10240), flag (54), and the
+// step's tag (55..63; a slot is rewritten two steps later at the earliest).
+__device__ __forceinline__ u64 anneal_pack(const ResOut& b, int step)
+{
+  return b.sum | (u64)(u32)b.diam << 40 | (u64)(b.flags & 1) << 54 | (u64)((step + 1) & 511) << 55;
 }
 
 template <int WB>
@@ -2760,9 +2779,7 @@ __global__ __launch_bounds__(1024) void k_anneal(AnnealArgs a)
   extern __shared__ __attribute__((aligned(16))) u32 lds[];
   __shared__ __attribute__((aligned(16))) u32 s_part[2][16];
   __shared__ int s_mv[5], s_dec[3];
-  __shared__ u64 s_sum;
-  __shared__ int s_diam, s_flags;
-  __shared__ AnnealState S;          // the chain's state; only thread 0 reads or writes it
+  __shared__ AnnealState S;          // the chain's state; only wave 0 reads or writes it
   const int tid = threadIdx.x, nth = blockDim.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   if (tid < 32 && (tid & 15) >= (nth + 63) / 64) s_part[tid >> 4][tid & 15] = 0;
@@ -2780,95 +2797,95 @@ __global__ __launch_bounds__(1024) void k_anneal(AnnealArgs a)
   T.s = 1; T.graph = 0; T.wb = WB; T.dq = (max(deg, 1) + 3) / 4;
   T.deg = deg; T.walk = 0;                            // res_run below is built without walks
   for (int k = 0; k < a.steps; k++) {                 // uniform: every exit below is uniform
-    if (tid == 0) {
+    if (wave == 0) {                                  // every lane holds the same values
+      uint64_t rng[4] = {S.rng[0], S.rng[1], S.rng[2], S.rng[3]};
       int found = 0, ma = 0, mb = 0, mc = 0, md = 0;
       for (int tries = 0; tries < 1000000 && !found; tries++) {
-        const int x = (int)anneal_rnd(S.rng, (u32)n), y = (int)anneal_rnd(S.rng, (u32)n);
-        const int bx = tab[x * dp + anneal_rnd(S.rng, (u32)deg)];
-        const int dy = tab[y * dp + anneal_rnd(S.rng, (u32)deg)];
+        const int x = (int)anneal_rnd(rng, (u32)n), y = (int)anneal_rnd(rng, (u32)n);
+        const u32 jx = anneal_rnd(rng, (u32)deg), jy = anneal_rnd(rng, (u32)deg);
+        const int bx = tab[x * dp + jx], dy = tab[y * dp + jy];
         if (x == y || x == dy || bx == y || bx == dy) continue;
-        if (anneal_has(tab, dp, deg, x, y) || anneal_has(tab, dp, deg, bx, dy)) continue;
-        anneal_swap(tab, dp, deg, x, bx, y, dy);
+        if (anneal_find(tab, dp, deg, x, y, lane) >= 0 || anneal_find(tab, dp, deg, bx, dy, lane) >= 0) continue;
+        anneal_swap(tab, dp, deg, x, bx, y, dy, lane);
         found = 1; ma = x; mb = bx; mc = y; md = dy;
       }
+      S.rng[0] = rng[0]; S.rng[1] = rng[1]; S.rng[2] = rng[2]; S.rng[3] = rng[3];
+      if (!found) S.stop = 1;
       s_mv[0] = found; s_mv[1] = ma; s_mv[2] = mb; s_mv[3] = mc; s_mv[4] = md;
     }
     __syncthreads();
-    if (!s_mv[0]) {
-      if (tid == 0) S.stop = 1;
-      break;
-    }
+    if (!s_mv[0]) break;
     const ResOut b = res_run<WB, false, false>(T, bits, s_part, tid, nth, wave);   // no walks (measured faster)
-    const int par = k & 1;                             // slots of this step (k is uniform; S.steps is thread 0's)
-    if (tid == 0) {
-      a.slots[par * G + g] = b;
-      __threadfence();
-      atomicAdd(a.bar, 1u);
-      const u32 target = (u32)G * (u32)(k + 1);
-      unsigned long long spins = 0;
-      int abort = 0;
-      while (__hip_atomic_load(a.bar, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) < target) {
-        __builtin_amdgcn_s_sleep(2);
-        if (++spins > ANNEAL_SPIN_LIMIT) { atomicOr(&a.st->err, 1); abort = 1; break; }
-      }
-      s_dec[2] = abort;
-    }
-    __syncthreads();
-    if (s_dec[2]) break;
-    // every block's totals, added in the same order in every workgroup
     if (wave == 0) {
-      u64 sum = 0;
-      int diam = 0;
-      u32 flags = 0;
-      for (int i = lane; i < G; i += 64) {
-        const ResOut* p = a.slots + par * G + i;
-        sum += __hip_atomic_load(&p->sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        diam = max(diam, __hip_atomic_load(&p->diam, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-        flags |= __hip_atomic_load(&p->flags, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      // publish this block's totals, then watch for every block's; they are
+      // added in the same order in every workgroup
+      u64* slots = a.slots + (k & 1) * G;
+      __hip_atomic_store(&slots[g], anneal_pack(b, k), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      u64 sum = 0, spins = 0;
+      u32 diam = 0, flags = 0;
+      int abort = 0;
+      for (int i0 = 0; i0 < G && !abort; i0 += 64) {
+        const int i = min(i0 + lane, G - 1);
+        u64 v;
+        for (;;) {
+          v = __hip_atomic_load(&slots[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (__ballot((int)(v >> 55) != ((k + 1) & 511)) == 0) break;
+          if (++spins > ANNEAL_SPIN_LIMIT) { abort = 1; break; }
+          __builtin_amdgcn_s_sleep(1);
+        }
+        if (i0 + lane < G) {
+          sum += v & ((1ull << 40) - 1);
+          diam = max(diam, (u32)(v >> 40) & 0x3fff);
+          flags |= (u32)(v >> 54) & 1;
+        }
       }
-      sum = wave_sum(sum); diam = wave_max(diam); flags = wave_or(flags);
-      if (lane == 0) { s_sum = sum; s_diam = diam; s_flags = (int)flags; }
+      if (abort) {
+        if (lane == 0) atomicOr(&a.st->err, 1);
+      } else {
+        sum = (u64)wave_sum_dpp((u32)(sum & 0xffffff)) + ((u64)wave_sum_dpp((u32)(sum >> 24)) << 24);
+        diam = (u32)wave_max((int)diam);
+        const bool disc = __ballot(flags != 0) != 0;
+        // the result as ODP_Set_aspl reports it (aspl.c:73-74, 332-336)
+        long lsum = (long)n * (n - 1) + (long)sum;
+        int d = max(1, (int)diam);
+        if (disc) d = n + 1;
+        double aspl = lsum / (((double)n - 1) * n);
+        lsum /= 2.0;
+        if (d > n) { d = INT_MAX; lsum = LONG_MAX; aspl = DBL_MAX; }
+        S.steps++;
+        int improved = 0, accept;
+        if (d < S.best_d || (d == S.best_d && aspl < S.best_a)) {
+          improved = 1;
+          S.best_d = d; S.best_sum = lsum; S.best_a = aspl;
+          if (d == S.low_d && aspl == S.low_a) S.optimum = 1;
+        }
+        if (S.optimum) accept = 1;              // the loop ends here; the move stays
+        else if (S.hill) accept = aspl <= S.cur_a;
+        else if (d < S.cur_d && !S.prio) accept = 1;
+        else if (d > S.cur_d && !S.prio) accept = 0;
+        else if (aspl <= S.cur_a) accept = 1;
+        else {
+          const double diff = (S.cur_a - aspl) * n * (n - 1);
+          const double u = ((double)(anneal_next(S.rng) >> 11) + 0.5) / 9007199254740992.0;
+          accept = exp(diff / S.temp) > u;
+        }
+        if (!S.optimum) {
+          if (accept) { S.cur_d = d; S.cur_a = aspl; S.accepted++; }
+          S.temp *= S.cooling;
+        }
+        s_dec[0] = improved; s_dec[1] = accept;
+      }
+      s_dec[2] = abort | 2 * S.optimum;
     }
     __syncthreads();
-    if (tid == 0) {
-      // the result as ODP_Set_aspl reports it (aspl.c:73-74, 332-336)
-      long lsum = (long)n * (n - 1) + (long)s_sum;
-      int d = max(1, s_diam);
-      if (s_flags & 1) d = n + 1;
-      double aspl = lsum / (((double)n - 1) * n);
-      lsum /= 2.0;
-      if (d > n) { d = INT_MAX; lsum = LONG_MAX; aspl = DBL_MAX; }
-      S.steps++;
-      int improved = 0, accept;
-      if (d < S.best_d || (d == S.best_d && aspl < S.best_a)) {
-        improved = 1;
-        S.best_d = d; S.best_sum = lsum; S.best_a = aspl;
-        if (d == S.low_d && aspl == S.low_a) S.optimum = 1;
-      }
-      if (S.optimum) accept = 1;              // the loop ends here; the move stays
-      else if (S.hill) accept = aspl <= S.cur_a;
-      else if (d < S.cur_d && !S.prio) accept = 1;
-      else if (d > S.cur_d && !S.prio) accept = 0;
-      else if (aspl <= S.cur_a) accept = 1;
-      else {
-        const double diff = (S.cur_a - aspl) * n * (n - 1);
-        const double u = ((double)(anneal_next(S.rng) >> 11) + 0.5) / 9007199254740992.0;
-        accept = exp(diff / S.temp) > u;
-      }
-      if (!S.optimum) {
-        if (accept) { S.cur_d = d; S.cur_a = aspl; S.accepted++; }
-        S.temp *= S.cooling;
-      }
-      s_dec[0] = improved; s_dec[1] = accept;
+    if (s_dec[2] & 1) break;
+    if (s_dec[0]) {                                    // the best graph: workgroup 0's table
+      if (g == 0)
+        for (int i = tid; i < n * deg; i += nth) a.best[i] = tab[(i / deg) * dp + (i % deg)];
+      __syncthreads();
     }
-    __syncthreads();
-    if (s_dec[0] && g == 0)                            // the best graph: workgroup 0's table
-      for (int i = tid; i < n * deg; i += nth) a.best[i] = tab[(i / deg) * dp + (i % deg)];
-    __syncthreads();
-    if (!s_dec[1] && tid == 0) anneal_swap(tab, dp, deg, s_mv[1], s_mv[3], s_mv[2], s_mv[4]);   // undo
-    if (tid == 0) s_dec[2] = S.optimum;               // thread 0's state decides, for every thread
-    __syncthreads();
-    if (s_dec[2]) break;
+    if (!s_dec[1] && wave == 0) anneal_swap(tab, dp, deg, s_mv[1], s_mv[3], s_mv[2], s_mv[4], lane);   // undo
+    if (s_dec[2] & 2) break;                           // the lower bounds were reached
   }
   __syncthreads();
   if (g == 0) {
