@@ -80,6 +80,19 @@ __device__ __forceinline__ void list_append(const LvList& lst, bool unsat, u64 v
   }
 }
 
+// the wave's sum, by adds between lanes (DPP: no LDS trips, as shuffles make);
+// the same value in every lane, in a scalar register
+__device__ __forceinline__ u32 wave_sum_dpp(u32 v)
+{
+  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);   // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);   // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);   // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);   // row_bcast:15
+  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);   // row_bcast:31
+  return (u32)__builtin_amdgcn_readlane((int)v, 63);
+}
+
 __device__ __forceinline__ u64 wave_sum(u64 v)
 {
 #pragma unroll
@@ -1624,7 +1637,8 @@ __global__ void k_tile_plan(const LevelTask* __restrict__ tasks, int ntasks, int
 // Bound by LDS reads (10.8 cycles a 16-byte neighbour read of a wave, conflicts
 // included); with two region copies and one workgroup a CU, nothing ran while a
 // unit was loaded, written back or waited at a barrier, 16 us a unit against the
-// 8 its reads take.  256 x 256 grid, d = 8: 144 -> 122 us a launch.
+// 8 its reads take.  256 x 256 grid, d = 8: 144 -> 122 us a launch, 118 with the
+// offsets of cells outside a level's window read from one row and the gains added between lanes.
 
 // cell (lx, ly) of the region of a tile: thread tid owns (wave + waves m, lane),
 // a wave whole region columns
@@ -1695,15 +1709,26 @@ __global__ __launch_bounds__(TILE_THREADS(DP), 4) void k_tile(const LevelTask* _
         usv = usv || (rid[m] >= 0 && !(val[m].x == f0 && val[m].y == f1));
       }
     }
-    auto offsets = [&](int m, u32* w) {
-      // (a cell outside the grid reads row 0's: it is never updated)
-      const uint2* o = (const uint2*)(g.toff + (int64_t)max(rid[m], 0) * DP);
+    // cell m's offsets; a cell outside the grid or not in [lo, hi) reads row 0's
+    // (it is not updated): one line instead of a line every four cells
+    auto offsets = [&](int m, u32* w, int lo, int hi) {
+      const int lx = wave + m * NW;
+      const bool in = rid[m] >= 0 && lx >= lo && lx < hi && lane >= lo && lane < hi;
+      const unsigned short* o = (const unsigned short*)g.toff + (int64_t)(in ? rid[m] : 0) * DP;
+      if constexpr (DP % 8 == 0) {
 #pragma unroll
-      for (int j = 0; j < DP / 4; j++) { const uint2 v = o[j]; w[2 * j] = v.x; w[2 * j + 1] = v.y; }
+        for (int j = 0; j < DP / 8; j++) {
+          const uint4 v = ((const uint4*)o)[j];
+          w[4 * j] = v.x; w[4 * j + 1] = v.y; w[4 * j + 2] = v.z; w[4 * j + 3] = v.w;
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < DP / 4; j++) { const uint2 v = ((const uint2*)o)[j]; w[2 * j] = v.x; w[2 * j + 1] = v.y; }
+      }
     };
     if (!ONE)
 #pragma unroll
-      for (int m = 0; m < PER; m++) offsets(m, off[ONE ? 0 : m]);
+      for (int m = 0; m < PER; m++) offsets(m, off[ONE ? 0 : m], g.lmax, TILE_RW - g.lmax);
     // a region whose cells are all zero, or all saturated, stays so for the k
     // levels: its tile is written back as loaded without running them (most
     // units of a first launch, and tiles the BFS front has just left)
@@ -1728,10 +1753,10 @@ __global__ __launch_bounds__(TILE_THREADS(DP), 4) void k_tile(const LevelTask* _
       u64x2 nx[ONE ? PER : 1];
       const int lo = (i + 1) * g.lmax, hi = TILE_RW - lo;
       u32 gain = 0;                                  // at most 8 * 128 bits a thread
-      if (ONE) offsets(0, off[0]);
+      if (ONE) offsets(0, off[0], lo, hi);
 #pragma unroll
       for (int m = 0; m < PER; m++) {
-        if (ONE && m + 1 < PER) offsets(m + 1, off[ONE ? (m + 1) & 1 : 0]);
+        if (ONE && m + 1 < PER) offsets(m + 1, off[ONE ? (m + 1) & 1 : 0], lo, hi);
         const int lx = wave + m * NW, sl = lx * TILE_RW + lane;
         if (rid[m] >= 0 && lx >= lo && lx < hi && lane >= lo && lane < hi) {
           const u64x2 o = src[sl];
@@ -1765,7 +1790,7 @@ __global__ __launch_bounds__(TILE_THREADS(DP), 4) void k_tile(const LevelTask* _
           if (rid[m] >= 0 && lx >= lo && lx < hi && lane >= lo && lane < hi) dst[lx * TILE_RW + lane] = nx[ONE ? m : 0];
         }
       }
-      const u64 wgain = wave_sum((u64)gain);
+      const u32 wgain = wave_sum_dpp(gain);
       if (lane == 0) red[wave][i] = wgain;
       if (i == 0 && tid == 0) claim_s = claim;
       __syncthreads();                               // level i is in LDS
@@ -2212,19 +2237,6 @@ __device__ __forceinline__ u64 uniform_u64(u64 v)
   const u32 lo = __builtin_amdgcn_readfirstlane((u32)v);
   const u32 hi = __builtin_amdgcn_readfirstlane((u32)(v >> 32));
   return ((u64)hi << 32) | lo;
-}
-
-// the wave's sum, by adds between lanes (DPP: no LDS trips, as shuffles make);
-// the same value in every lane, in a scalar register
-__device__ __forceinline__ u32 wave_sum_dpp(u32 v)
-{
-  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, false);   // row_shr:1
-  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, false);   // row_shr:2
-  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, false);   // row_shr:4
-  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, false);   // row_shr:8
-  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);   // row_bcast:15
-  v += __builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);   // row_bcast:31
-  return (u32)__builtin_amdgcn_readlane((int)v, 63);
 }
 
 // part: 16 words a wave each, those past the workgroup's waves zero
