@@ -1057,7 +1057,7 @@ __global__ __launch_bounds__(PG_WG) void k_pgather(const LevelTask* __restrict__
     }
     lds_barrier();
     // the unit's rows: written, counted, listed; wave w takes rows [64 w, 64 w + 64)
-    u64 pop = 0;
+    u32 pop = 0;                                    // at most 64 rows of 1024 bits a wave
     // the lane's addresses of this part are computed here: hoisted out of the
     // unit loop they would take the registers of the gathers in flight
     int lane = lane_;
@@ -1077,14 +1077,14 @@ __global__ __launch_bounds__(PG_WG) void k_pgather(const LevelTask* __restrict__
             u64v2 o; o.x = v.x; o.y = v.y;
             row_store<NT>(o, (u64v2*)(nxt + (int64_t)r * 16 + w));
           }
-          pop += (u64)(__popcll(v.x) + __popcll(v.y));
+          pop += (u32)(__popcll(v.x) + __popcll(v.y));
         }
         if (LS) list_append(lst, valid && !(v.x == f0 && v.y == f1), ((u64)t << 48) | ((u64)r << 24) | (u64)w, v.x, v.y);
       }
     }
     if (count) {
-      pop = wave_sum(pop);
-      if (lane == 0) s_pop[wave] = pop;
+      const u32 sum = wave_sum_dpp(pop);
+      if (lane == 0) s_pop[wave] = sum;
     }
     lds_barrier();                                  // acc is read, s_pop written
     if (count && tid == 0) {
