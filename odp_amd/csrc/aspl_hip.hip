@@ -1256,6 +1256,7 @@ struct Evaluator {
   struct LvState {
     int K = 0, L1 = 1, nzero = 0, be0 = 2;
     bool fr = false;                    // frontier-mode level kernel (graphs with many levels)
+    int fr_from = 1;                    // ... from this level on (every row of it; >= L1)
     int tk = 0;                         // k_tile levels per launch (0: one k_level launch per level)
     int tside = TILE_MIN;               // k_tile's tile side (halo = (64 - side) / 2)
     bool thin = false;                  // the level before spec runs thin
@@ -1412,7 +1413,7 @@ struct Evaluator {
           : (r.urow ? (r.batch == 16 ? k_level<true, 16, false, false> : r.batch == 8 ? k_level<true, 8, false, false> : k_level<true, 4, false, false>)
                     : (r.batch == 16 ? k_level<false, 16, false, false> : r.batch == 8 ? k_level<false, 8, false, false> : k_level<false, 4, false, false>));
       hipLaunchKernelGGL(kern, dim3(grid), dim3(LEVEL_WG), 0, st,
-                         r.tasks + lv.first, r.wg_start, lv.cnt_t, L, RING, r.upw, r.xcd, lv.L1, mode, lst);
+                         r.tasks + lv.first, r.wg_start, lv.cnt_t, L, RING, r.upw, r.xcd, lv.fr_from, mode, lst);
     }
     HIPC(hipGetLastError());
     timed_end(tl);
@@ -1471,7 +1472,7 @@ struct Evaluator {
   {
     LevelRun& r = lr;
     lv.cnt_t = std::min(r.group, r.ntasks - lv.first);
-    lv.launched = lv.L1; lv.examined = 0; lv.running = lv.cnt_t;
+    lv.launched = lv.L1; lv.examined = 0; lv.running = lv.cnt_t; lv.fr_from = lv.L1;
     lv.batch_end = lv.first == 0 ? lv.be0 : first_batch_end();
     // the last evaluation ended at level batch_end - 1: expect the same, and
     // launch that level count-only (timed passes keep every level whole)
@@ -1597,11 +1598,15 @@ struct Evaluator {
                 ? std::min(TILE_KMAX, halo / std::max(1, geo_lmax)) : 0;
     lv.be0 = first_batch_end();
     // frontier mode pays off over long level sequences; with few levels every
-    // level is dense and the plain kernel is faster
-    lv.fr = !lv.tk && (guess_levels == 0 || guess_levels > FRONTIER_MIN_LEVELS);
+    // level is dense and the plain kernel is faster.  Without a last evaluation
+    // to tell, a plan with row parts runs its own levels and goes over when
+    // FRONTIER_MIN_LEVELS of them were not enough (lv_step): a frontier level of
+    // n = 65536, d = 16 takes 500 us, the row parts' 447; serving's first requests of
+    // nine chains 14.3 -> 10.4 ms
+    lv.fr = !lv.tk && (guess_levels == 0 ? r.parts == 0 : guess_levels > FRONTIER_MIN_LEVELS);
     if (thin_k > 0 && thin_k != r.thin) { r.thin = thin_k; pl_fresh = false; }
     lv.plfresh = lv.fresh && pl_fresh;
-    lv.check = (lv.fr || (pg_on() && r.fold)) && !(lv.fresh && asym_fresh);
+    lv.check = (lv.fr || (!lv.tk && guess_levels == 0) || (pg_on() && r.fold)) && !(lv.fresh && asym_fresh);
     lv.graphed = r.group == r.ntasks && use_graph(lv_key(lv.be0));
     if (!lv.graphed) lv_prepare();
     lv.sts.assign(r.ntasks, LvTask{1, 0, 0, 0});
@@ -1658,6 +1663,10 @@ struct Evaluator {
       lv.spec = -1;
     }
     if (lv.running > 0 && lv.launched < n) {
+      if (guess_levels == 0 && !lv.tk && !lv.fr && lv.launched >= FRONTIER_MIN_LEVELS) {
+        lv.fr = true;
+        lv.fr_from = lv.launched;
+      }
       const int step = std::min(batch_cap, std::min(MAX_BATCH_LEVELS, std::max(lv.launched, 8)));
       lv.batch_end = lv.tk ? tile_batch_end(lv.launched, step) : capped_end(std::min(n, lv.launched + step));
       if (batch_cap < MAX_BATCH_LEVELS && spec_at(lv.batch_end)) {
@@ -1739,7 +1748,7 @@ struct Evaluator {
         // (unless the launch only counts) written once, the neighbour ids once per launch
         for (int t = first; t < first + cnt_t; t++)
           if (tl.level <= stv[t].lwork) {
-            const double share = lv.fr || lv.tk
+            const double share = (lv.fr && tl.level >= lv.fr_from) || lv.tk
                                      ? (double)r.h_acnt[(size_t)(tl.level % RING) * r.ntasks + t] / ((double)n * r.segs)
                                      : 1.0;
             bytes += share * tl.nlev * (double)n * ((avg_deg + 1.0 + tl.wr) * ((r.l[t] + 63) / 64) * 8.0 + 4.0 * avg_deg);
