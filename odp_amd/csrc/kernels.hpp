@@ -2440,11 +2440,15 @@ __device__ __forceinline__ ResOut res_run(const ResTask& T, u32* cur, u32 (*s_pa
         row_or2<WB>(own[i], cbase, v0.x); row_or2<WB>(own[i], cbase, v0.y);
         if (T.dq > 1) { row_or2<WB>(own[i], cbase, v0.z); row_or2<WB>(own[i], cbase, v0.w); }
         if (T.dq > 2 && !(STOP && is_full(own[i]))) {        // STOP: a row filled by 8 neighbours reads no more
+          uint4 v2 = make_uint4(0, 0, 0, 0);           // ids past the sixteenth: a group ahead
+          if (T.dq > 4) v2 = ids_at(i, nl)[2];
           row_or2<WB>(own[i], cbase, v1.x); row_or2<WB>(own[i], cbase, v1.y);
           if (T.dq > 3) { row_or2<WB>(own[i], cbase, v1.z); row_or2<WB>(own[i], cbase, v1.w); }
-          for (int j = 4; j < T.dq && !(STOP && is_full(own[i])); j++) {
-            const uint2 v = ((const uint2*)ids_at(i, nl))[j];
+          for (int j = 4; j < T.dq && !(STOP && is_full(own[i])); j += 2) {
+            const uint4 v = v2;
+            if (j + 2 < T.dq) v2 = ids_at(i, nl)[(j >> 1) + 1];
             row_or2<WB>(own[i], cbase, v.x); row_or2<WB>(own[i], cbase, v.y);
+            if (j + 1 < T.dq) { row_or2<WB>(own[i], cbase, v.z); row_or2<WB>(own[i], cbase, v.w); }
           }
         }
       }
