@@ -54,8 +54,12 @@ static const double LIST_MAX_FRAC_PG = 1.0 / 32; // ... by k_pgather, whose coun
 static const int LV_MISS_LEVELS = 64;            // levels whose missing pairs an evaluation records
 // adjacency tables up to this size reach the device through the resident
 // plan's table build reading pinned host memory (one kernel instead of a DMA
-// command plus the kernel); larger ones are copied by DMA
-static const size_t ZC_MAX_BYTES = 256u << 10;
+// command plus the kernel); larger ones are copied by DMA.  The kernel reads
+// the link as fast as the copy and saves its command: an evaluation of n = 8192,
+// d = 12 (384 KiB) 67.2 -> 53.0 us, 16384, 16 (1 MiB) 124 -> 108, 40000, 16
+// (2.5 MiB) 538 -> 530.  A symmetric graph's build reads the base table once per
+// copy of it and again for the device's: the smaller limit
+static const size_t ZC_MAX_BYTES = 4096u << 10, ZC_MAX_BYTES_SYM = 256u << 10;
 static const size_t LMAX_HOST_ENTRIES = 8192;   // adjacency entries whose longest edge the host measures itself
 static const int TILE_MIN = 32;                 // smallest tile side of k_tile (halo 16)
 static const int SPARSE_GRID = 2048;            // workgroups of a k_sparse launch (8 per CU)
@@ -825,7 +829,8 @@ struct Evaluator {
     stage_is_device = true;
     mirror_ok = false;
     memcpy(h_stage, adjacency, sizeof(int) * adj_elems());
-    if (plan.plan == ODPX_PLAN_RESIDENT && !ext_adj && sizeof(int) * adj_elems() <= ZC_MAX_BYTES) {
+    if (plan.plan == ODPX_PLAN_RESIDENT && !ext_adj &&
+        sizeof(int) * adj_elems() <= (s == 1 && !grid_s ? ZC_MAX_BYTES : ZC_MAX_BYTES_SYM)) {
       adj_on_host = true;          // the next table build reads it from host memory
     } else {
       adj_on_host = false;
