@@ -62,7 +62,10 @@ struct LvList {
 // shared helpers
 
 // appends the wave's lanes with `unsat` set to the workgroup's sub-list: one
-// atomic per wave.  Called by whole waves.
+// atomic per wave.  Called by whole waves.  V: with the chunks' bits, where the
+// list takes them.  k_level's lists never do, and it has an instance without the
+// branch: four registers fewer, a listing level of n = 22000, d = 64 in 0.27 instead of 0.39 ms
+template <bool V>
 __device__ __forceinline__ void list_append(const LvList& lst, bool unsat, u64 val, u64 x = 0, u64 y = 0)
 {
   const u64 m = __ballot(unsat);
@@ -75,7 +78,7 @@ __device__ __forceinline__ void list_append(const LvList& lst, bool unsat, u64 v
     const u32 e = b + (u32)__popcll(m & ((1ULL << lane) - 1));
     if (e < lst.cap) {
       lst.e[(u64)sub * lst.cap + e] = val;
-      if (lst.v) { u64x2 o; o.x = x; o.y = y; lst.v[(u64)sub * lst.cap + e] = o; }
+      if (V && lst.v) { u64x2 o; o.x = x; o.y = y; lst.v[(u64)sub * lst.cap + e] = o; }
     }
   }
 }
@@ -577,7 +580,7 @@ __global__ __launch_bounds__(LEVEL_WG) void k_level(const LevelTask* __restrict_
         }
       }
     }
-    if (LS) list_append(lst, unsat, ((u64)t << 48) | ((u64)q.r << 24) | (u64)q.w);   // a slot per unsaturated chunk
+    if (LS) list_append<false>(lst, unsat, ((u64)t << 48) | ((u64)q.r << 24) | (u64)q.w);   // a slot per unsaturated chunk
   }
   if (!count) return;
   pop = wave_sum(pop);
@@ -1092,7 +1095,7 @@ __global__ __launch_bounds__(PG_WG) void k_pgather(const LevelTask* __restrict__
           }
           pop += (u32)(__popcll(v.x) + __popcll(v.y));
         }
-        if (LS) list_append(lst, valid && !(v.x == f0 && v.y == f1), ((u64)t << 48) | ((u64)r << 24) | (u64)w, v.x, v.y);
+        if (LS) list_append<true>(lst, valid && !(v.x == f0 && v.y == f1), ((u64)t << 48) | ((u64)r << 24) | (u64)w, v.x, v.y);
       }
     }
     if (count) {
@@ -1440,7 +1443,7 @@ __global__ __launch_bounds__(LEVEL_WG) void k_thin(const LevelTask* __restrict__
     }
     add_gains(tasks, level, ring, t, -miss);
     if (fold) add_gains(tasks, level, ring, t2, t2 == t ? 0 : -miss);
-    list_append(lst2, unsat, id, x.x, x.y);
+    list_append<true>(lst2, unsat, id, x.x, x.y);
   }
 }
 
