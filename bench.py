@@ -709,9 +709,10 @@ def main():
                 "launches": st[pre + "_launches"], "measured_traffic": measured,
                 "work_equivalent": {"GBs": round(alg / (launch_ms * 1e-3) / 1e9, 1) if launch_ms > 0 else 0.0,
                                     "bytes_per_launch": alg,
-                                    "note": "operand bytes of next[v] = cur[v] | OR cur[u] (rows * ((d+2)*k*8 "
-                                            "+ 4d) per level), most of them served by L2/MALL; a work rate, "
-                                            "not an HBM fraction"},
+                                    "note": "operand bytes of next[v] = cur[v] | OR cur[u] for the rows a "
+                                            "level gathers for (about half of them in folded levels), and the "
+                                            "rows written, most of them served by L2/MALL; a work rate, not an "
+                                            "HBM fraction"},
                 "timed_steps_ms_per_step": round(1e3 * el_live / args.steps, 4)}
     if kern == "k_resident_w":
         roofline["note"] = ("the bit rows live in LDS: HBM carries the neighbour ids only; the kernel is bound "

@@ -134,7 +134,11 @@ typedef struct {
   double    eval_ms;          /* wall time of those evaluations (host clock)       */
   long long level_launches;   /* gather-level launches that did work               */
   double    level_ms;         /* their summed duration, HIP events on the launch stream */
-  double    level_bytes;      /* their algorithmic bytes: rows*((d+2)*k*8 + 4d)     */
+  double    level_bytes;      /* their algorithmic bytes: rows*(s*((d+1)*k*8 + 4d) + k*8),
+                                 s the share of the rows a launch gathers for ((T+1)/(2T)
+                                 in a folded level of T blocks, else 1), d the neighbours
+                                 it takes (a part of them in a thin level), the last
+                                 term only for rows that are written                */
   double    level_min_bytes;  /* their compulsory bytes: every row of a working block
                                  read once and (unless count-only) written once,
                                  rows*k*8*(1 + written), plus the ids once per launch */

@@ -310,8 +310,9 @@ static u32 list_cap_env()
 // kernel timing: HIP events recorded on the launch stream around launches
 
 enum { T_OTHER = 0, T_LEVEL = 1, T_RESIDENT = 2 };
-// nlev: levels the launch runs; wr: it writes the rows (0: a count-only level)
-struct TimedLaunch { hipEvent_t a, b; int kind, level, nlev = 1, wr = 1; };
+// nlev: levels the launch runs; wr: it writes the rows (0: a count-only level);
+// fold: folded if the table is symmetric; nbrs: neighbours a row takes (-1: all)
+struct TimedLaunch { hipEvent_t a, b; int kind, level, nlev = 1, wr = 1; bool fold = false; int nbrs = -1; };
 static bool g_stats_on = false;
 static bool g_stats_live = false;       // timed evaluations keep the untimed launch sequence
 static ODPX_Stats g_stats;
@@ -375,7 +376,7 @@ struct LevelRun {
   int thin = 0;                         // neighbours the pair lists mark thin
   u64x2* list_v = nullptr;
   u64* list2 = nullptr; u64x2* list2_v = nullptr;
-  u64* h_acnt = nullptr;                // processed-unit counts on the host (kernel timing only)
+  u64* h_acnt = nullptr;                // processed-unit counts on the host, then the asymmetry flag (kernel timing only)
   size_t flag_bytes = 0;
   // part-phased gather (k_pgather): row parts, sorted neighbour runs, persistent grid
   int parts = 0, psp = 0, pgrid = 0, pupt = 0;
@@ -1051,7 +1052,7 @@ struct Evaluator {
       dalloc(&r.cnt, (size_t)3 * RING * ntasks);     // counts, changed, processed
       // done flags, the lists' counters (all cleared by the preparation), the table's asymmetry flag
       dalloc(&r.done, (size_t)ntasks + LIST_COUNTERS + 1);
-      hfree(&r.h_acnt); halloc(&r.h_acnt, (size_t)RING * ntasks);
+      hfree(&r.h_acnt); halloc(&r.h_acnt, (size_t)RING * ntasks + 1);
       dalloc(&r.tasks, (size_t)ntasks); dalloc(&r.wg_start, (size_t)ntasks + 1);
       halloc_coherent(&r.h_cnt, &r.h_cnt_dev, (size_t)RING * ntasks);
       r.task_cap = ntasks;
@@ -1270,6 +1271,7 @@ struct Evaluator {
     bool pend_fin = false;              // the enqueued batch ends with k_lvfin (sequence number lvseq)
     bool fresh = false, plfresh = false; // the preparation keeps the table / the pair lists
     bool check = false;                  // ... and checks the table's symmetry
+    int asym = -1;                       // whether it is not symmetric (where folded levels ask; -1: not handed over)
     int first = 0, cnt_t = 0;
     int launched = 0, examined = 0, running = 0, batch_end = 0;
     std::vector<LvTask> sts;
@@ -1386,6 +1388,8 @@ struct Evaluator {
     const LvList lst2{r.list2, r.list_n + LIST_SUBS * LIST_PAD, std::min(r.list_cap, THIN2_CAP / LIST_SUBS), r.list2_v};
     TimedLaunch tl;
     tl.wr = (mode & LV_STORE) ? 1 : 0;
+    tl.fold = asym != nullptr;
+    tl.nbrs = (mode & LV_THIN) ? r.thin : -1;
     // k_sparse is timed apart: its work is the listed chunks, not a level
     timed_begin(tl, (mode & LV_SPARSE) ? T_OTHER : T_LEVEL, L, st);
     if (thin && (mode & LV_SPARSE)) {
@@ -1459,7 +1463,7 @@ struct Evaluator {
     LevelRun& r = lr;
     if (lv_fin_ok(lv.examined, to)) {
       hipLaunchKernelGGL(k_lvfin, dim3(1), dim3(256), 0, st, r.cnt, r.ntasks, lv.examined, to, RING, r.h_cnt_dev,
-                         d_err, lvh_dev, d_lvseq);
+                         d_err, r.asym, lvh_dev, d_lvseq);
       HIPC(hipGetLastError());
       note_fin(true);
       return;
@@ -1467,9 +1471,11 @@ struct Evaluator {
     note_fin(false);
     HIPC(hipMemcpyAsync(r.h_cnt, r.cnt, sizeof(u64) * RING * r.ntasks, hipMemcpyDeviceToHost, st));
     HIPC(hipMemcpyAsync(h_err, d_err, sizeof(int), hipMemcpyDeviceToHost, st));
-    if (timed())
+    if (timed()) {
       HIPC(hipMemcpyAsync(r.h_acnt, r.cnt + (size_t)2 * RING * r.ntasks, sizeof(u64) * RING * r.ntasks,
                           hipMemcpyDeviceToHost, st));
+      HIPC(hipMemcpyAsync(r.h_acnt + (size_t)RING * r.ntasks, r.asym, sizeof(u32), hipMemcpyDeviceToHost, st));
+    }
   }
 
   // the first levels and the first batch of group lv.first
@@ -1615,6 +1621,7 @@ struct Evaluator {
     lv.graphed = r.group == r.ntasks && use_graph(lv_key(lv.be0));
     if (!lv.graphed) lv_prepare();
     lv.sts.assign(r.ntasks, LvTask{1, 0, 0, 0});
+    lv.asym = -1;
     lv.any_disc = false;
     lv.max_d = 1; lv.lmax = 0;
     for (double& m : lv.miss) m = 0;
@@ -1722,6 +1729,8 @@ struct Evaluator {
     }
     if (!seen) HIPC(hipStreamSynchronize(st));
     if (lv.pend_fin) *h_err = lvh->err;
+    if (lr.fold && (lv.pend_fin || timed()))
+      lv.asym = (lv.pend_fin ? lvh->asym : *(const u32*)(lr.h_acnt + (size_t)RING * lr.ntasks)) != 0;
   }
 
   void run_level(u64* excess, int* diam, bool* disc)
@@ -1749,14 +1758,19 @@ struct Evaluator {
         double bytes = 0, minb = 0;
         // a level processes a share of the (row, segment) units: all of them, or
         // in frontier mode the active ones; bytes are that share of the full level's.
+        // A folded level gathers for the units of one of each pair across the diagonal
+        // and stores both; a thin one takes a part of the neighbours.
         // Compulsory bytes: each processed row of a working block read once and
         // (unless the launch only counts) written once, the neighbour ids once per launch
+        const double fold = tl.fold && lv.asym == 0 ? (r.ntasks + 1) / (2.0 * r.ntasks) : 1.0;
+        const double nbrs = tl.nbrs < 0 ? avg_deg : std::min((double)tl.nbrs, avg_deg);
         for (int t = first; t < first + cnt_t; t++)
           if (tl.level <= stv[t].lwork) {
             const double share = (lv.fr && tl.level >= lv.fr_from) || lv.tk
                                      ? (double)r.h_acnt[(size_t)(tl.level % RING) * r.ntasks + t] / ((double)n * r.segs)
                                      : 1.0;
-            bytes += share * tl.nlev * (double)n * ((avg_deg + 1.0 + tl.wr) * ((r.l[t] + 63) / 64) * 8.0 + 4.0 * avg_deg);
+            const double row = ((r.l[t] + 63) / 64) * 8.0;
+            bytes += share * tl.nlev * (double)n * (fold * ((nbrs + 1.0) * row + 4.0 * nbrs) + tl.wr * row);
             minb += share * (double)n * ((r.l[t] + 63) / 64) * 8.0 * (1.0 + tl.wr);
           }
         if (minb > 0) minb += (double)n * avg_deg * 4.0;

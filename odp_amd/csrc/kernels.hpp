@@ -2505,15 +2505,17 @@ __device__ __forceinline__ void res_commit(ResOut* out, int graph, const ResOut&
 // End of a batch of levels as the host reads it (pinned, coherent host memory).
 struct LvHost {
   int err;          // the device error flag as it stood at the end of the batch
-  u32 seq;          // the batch's sequence number, written after err and the counters
+  u32 asym;         // the table's asymmetry flag (k_symcheck)
+  u32 seq;          // the batch's sequence number, written after these and the counters
 };
 
-// The counters of levels [from, to) (ring slots L % ring of every task) and
-// the error flag, stored into host memory; then the next sequence number
+// The counters of levels [from, to) (ring slots L % ring of every task), the
+// error flag and the table's asymmetry flag, stored into host memory; then the next sequence number
 // (kept on the device, so that a replayed graph advances it too), which the
 // host watches for instead of synchronising the stream.
 __global__ __launch_bounds__(256) void k_lvfin(const u64* __restrict__ cnt, int ntasks, int from, int to, int ring,
-                                              u64* hcnt, const int* err, LvHost* host, u32* dseq)
+                                              u64* hcnt, const int* err, const u32* asym, LvHost* host,
+                                              u32* dseq)
 {
   const int m = (to - from) * ntasks;
   for (int i = threadIdx.x; i < m; i += blockDim.x) {
@@ -2525,6 +2527,7 @@ __global__ __launch_bounds__(256) void k_lvfin(const u64* __restrict__ cnt, int 
   __syncthreads();
   if (threadIdx.x == 0) {
     host->err = *err;
+    host->asym = *asym;
     const u32 sq = *dseq + 1;
     *dseq = sq;
     __threadfence_system();
