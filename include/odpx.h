@@ -157,6 +157,15 @@ typedef struct {
 void ODPX_Stats_enable(int on);
 void ODPX_Stats_reset(void);
 void ODPX_Stats_get(ODPX_Stats *out);
+/* Which ways evaluations went, counted from the library's load (timed or not). */
+typedef struct {
+  long long folded;      /* evaluations of ODP_Set_aspl and its like whose gather levels ran folded */
+  long long thin;        /* levels before the expected last one run over a part of the neighbours */
+  long long thin_whole;  /* ... run again over all of them: their lists were too short */
+  long long thin_late;   /* ... whose rows were written after all: the next level was not the last */
+  long long chunked;     /* ODPX_Batch_eval calls sent in chunks */
+} ODPX_Routes;
+void ODPX_Routes_get(ODPX_Routes *out);
 
 /* ---- batched evaluation ------------------------------------------------- */
 /* Uploads ngraphs general (s = 1) graphs, packed as for ODPX_Batch_eval, and

@@ -61,6 +61,15 @@ class Stats(ctypes.Structure):
         return {name: getattr(self, name) for name, _ in self._fields_}
 
 
+class Routes(ctypes.Structure):
+    """ODPX_Routes (include/odpx.h)."""
+    _fields_ = [("folded", ctypes.c_longlong), ("thin", ctypes.c_longlong), ("thin_whole", ctypes.c_longlong),
+                ("thin_late", ctypes.c_longlong), ("chunked", ctypes.c_longlong)]
+
+    def as_dict(self):
+        return {name: getattr(self, name) for name, _ in self._fields_}
+
+
 class Result(ctypes.Structure):
     """ODPX_Result (include/odpx.h)."""
     _fields_ = [("id", ctypes.c_longlong), ("chain", ctypes.c_int), ("status", ctypes.c_int),
@@ -142,6 +151,7 @@ def load():
     _sig(lib, "ODPX_Stats_enable", None, [_I])
     _sig(lib, "ODPX_Stats_reset", None, [])
     _sig(lib, "ODPX_Stats_get", None, [ctypes.POINTER(Stats)])
+    _sig(lib, "ODPX_Routes_get", None, [ctypes.POINTER(Routes)])
     batch_args = [_I, _P, _P, _P, _P, _P, _P, _P]
     _sig(lib, "ODPX_Batch_eval", _I, batch_args)
     _sig(lib, "ODPX_Batch_load", _I, [_I, _P, _P, _P, _P])
@@ -292,6 +302,13 @@ def stats():
     s = Stats()
     load().ODPX_Stats_get(ctypes.byref(s))
     return s.as_dict()
+
+
+def routes():
+    """ODPX_Routes_get: which ways evaluations went, counted from the library's load."""
+    r = Routes()
+    load().ODPX_Routes_get(ctypes.byref(r))
+    return r.as_dict()
 
 
 # ---- batched evaluation -----------------------------------------------------

@@ -316,6 +316,8 @@ struct TimedLaunch { hipEvent_t a, b; int kind, level, nlev = 1, wr = 1; bool fo
 static bool g_stats_on = false;
 static bool g_stats_live = false;       // timed evaluations keep the untimed launch sequence
 static ODPX_Stats g_stats;
+// the ways evaluations went that results do not show (ODPX_Routes_get)
+static struct { std::atomic<long long> folded{0}, thin{0}, thin_whole{0}, thin_late{0}, chunked{0}; } g_routes;
 static std::vector<hipEvent_t> g_evpool;
 static std::vector<TimedLaunch> g_pending;
 
@@ -1489,6 +1491,7 @@ struct Evaluator {
     // launch that level count-only (timed passes keep every level whole)
     lv.spec = spec_at(lv.batch_end) ? lv.batch_end - 1 : -1;
     lv.thin = listed_at(lv.spec) && pg_on() && thin_k > 0;
+    if (lv.thin) g_routes.thin++;
     if (lv.first == 0 && lv.graphed) {
       // prepare + the first levels + the first batch + the counter copies as one graph
       const int be = lv.batch_end, L1 = lv.L1;
@@ -1646,6 +1649,7 @@ struct Evaluator {
                            r.cnt + (size_t)(k % RING) * r.ntasks + lv.first, lv.cnt_t, (int*)nullptr, 0);
         HIPC(hipGetLastError());
       }
+      g_routes.thin_whole++;
       lv.spec = -1; lv.thin = false; thin_k = 0;
       lv_levels(L, lv.batch_end);
       return false;
@@ -1670,7 +1674,7 @@ struct Evaluator {
       // (after a thin level, that level's rows first)
       const bool thin = lv.thin;
       lv.thin = false;
-      if (thin) lv_launch(lv.spec - 1, LV_STORE);
+      if (thin) { g_routes.thin_late++; lv_launch(lv.spec - 1, LV_STORE); }
       lv_launch(lv.spec, LV_STORE);
       lv.spec = -1;
     }
@@ -1684,6 +1688,7 @@ struct Evaluator {
       if (batch_cap < MAX_BATCH_LEVELS && spec_at(lv.batch_end)) {
         lv.spec = lv.batch_end - 1;
         lv.thin = lv.launched < lv.spec && listed_at(lv.spec) && pg_on() && thin_k > 0;
+        if (lv.thin) g_routes.thin++;
       }
       lv_levels(lv.launched, lv.batch_end);
       lv.launched = std::max(lv.launched, lv.batch_end);
@@ -1710,6 +1715,7 @@ struct Evaluator {
     u64 tot = 0;
     for (const LvTask& q : lv.sts) tot += q.sum;
     *excess = tot; *diam = lv.max_d; *disc = lv.any_disc;
+    if (pg_on() && lv.asym == 0 && lv.launched > lv.L1) g_routes.folded++;
     if (timed()) flush_level_stats(lv.sts.data(), 0, 0);
   }
 
@@ -2653,6 +2659,11 @@ extern "C" void ODPX_Stats_enable(int on)
 }
 extern "C" void ODPX_Stats_reset(void) { memset(&g_stats, 0, sizeof g_stats); }
 extern "C" void ODPX_Stats_get(ODPX_Stats* out) { *out = g_stats; }
+extern "C" void ODPX_Routes_get(ODPX_Routes* out)
+{
+  out->folded = g_routes.folded; out->thin = g_routes.thin; out->thin_whole = g_routes.thin_whole;
+  out->thin_late = g_routes.thin_late; out->chunked = g_routes.chunked;
+}
 
 extern "C" int ODPX_Autotune(void* adjacency, int repeats)
 {
@@ -3189,6 +3200,7 @@ extern "C" int ODPX_Batch_eval(int ngraphs, const int* nodes, const int* degrees
     ODPX_Batch_load(ngraphs, nodes, degrees, offsets, packed);
     return ODPX_Batch_run(diameter, sum, ASPL);
   }
+  g_routes.chunked++;
   batch_shape(ngraphs, nodes, degrees, offsets);
   if (!B.copies) {
     HIPC(hipStreamCreateWithFlags(&B.copies, hipStreamNonBlocking));
