@@ -122,10 +122,16 @@ int  ODPX_Set_aspl_noalloc(int nodes, int degree, const int *adjacency, int *dia
 /* The kind ODP_Init_aspl_* picks: ODP_ASPL if set (MATRIX, MATRIX_SAVING, BFS;
  * unknown values exit as at Init), else MATRIX when the GPU memory estimate
  * of MATRIX is at most 2048 MB, MATRIX_SAVING otherwise (utils.c:1238-1266 with
- * is_cpu = false, procs = 1).  Returns 1 (MATRIX), 2 (MATRIX_SAVING) or 3 (BFS). */
+ * is_cpu = false, procs = 1).  Returns 1 (MATRIX), 2 (MATRIX_SAVING) or 3 (BFS).
+ * MATRIX_SAVING asked for by ODP_ASPL keeps 32 blocks of 1024 source columns on
+ * the device (2 x 32 x 128 bytes per vertex: 0.8 GB at 100000).  Chosen by size
+ * for a general graph, it keeps every block while that takes at most 16 GiB and
+ * an eighth of the free memory (nodes^2 / 4 bytes: 2.5 GB at 100000), which is
+ * faster; ODPX_Get_plan's group tells which (0: every block). */
 int    ODPX_Get_kind(int nodes, int degree, int has_num_degrees, int symmetries, int grid_s);
 /* The memory estimate in MB of that rule and of the ODP_PROFILE report
- * (utils.c:1206-1236 with is_cpu = false, procs = 1). */
+ * (utils.c:1206-1236 with is_cpu = false, procs = 1): the reference's buffers, not
+ * the blocks this library keeps (above). */
 double ODPX_Get_mem_usage(int kind, int nodes, int degree, int has_num_degrees, int symmetries, int grid_s);
 
 /* ---- kernel timing ------------------------------------------------------ */

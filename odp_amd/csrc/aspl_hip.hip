@@ -34,11 +34,13 @@
 static const int KIND_MATRIX = 1, KIND_SAVING = 2, KIND_BFS = 3;   // the reference's ASPL_* (common.h:39-41)
 static const int GPU_CHUNK_WORDS = 64;          // column-block width of MATRIX_SAVING (parameter.h:13)
 static const int SAVING_GROUP = 32;             // MATRIX_SAVING blocks resident at once (4 per XCD) ...
-static const size_t SAVING_BYTES = 16ull << 30;  // ... unless all blocks' buffers stay within this (and half the free
-                                                // memory): the folded levels need them all resident, and k_direct
-                                                // walks the rows once instead of once per group (n = 100000, d = 8:
-                                                // 4.99 -> 3.28 ms; n = 131072, d = 16: 10.8 -> 6.5 ms; n = 200000,
-                                                // d = 8, 10 GB: 28.4 -> 17.2 ms)
+// ... unless the kind is the size's own choice (ODP_ASPL not set: who asks for
+// MATRIX_SAVING asks for its bounded memory) and all blocks' buffers stay within
+// this and an eighth of the free memory (so that eight processes that look at
+// once all fit): the folded levels need them all resident, and k_direct walks the
+// rows once instead of once per group (n = 100000, d = 8, 2.5 GB instead of 0.8:
+// 4.99 -> 3.0 ms; n = 131072, d = 16: 10.8 -> 6.3 ms; n = 200000, d = 8, 10 GB: 28.4 -> 17.2 ms)
+static const size_t SAVING_BYTES = 16ull << 30;
 static const int LEVEL_BLOCK_WORDS = 16;        // default column-block width of the level plan
 static const int RES_WB_MAX = 8;                // widest resident block: 256 sources
 static const int BATCH_CLASSES = 5;             // size classes of the batch launch policy
@@ -910,7 +912,8 @@ struct Evaluator {
     // one XCD gathers from stay within a few MiB (its L2).  MATRIX
     // keeps every block resident and advances all of them per launch (the full
     // bit matrix, blocked); MATRIX_SAVING keeps SAVING_GROUP blocks resident
-    // at a time, bounding memory as the reference does (aspl.c:77-119).
+    // at a time, bounding memory as the reference does (aspl.c:77-119), where
+    // ODP_ASPL asks for it or all blocks would take too much (SAVING_BYTES).
     p.plan = ODPX_PLAN_LEVEL;
     int W = (nsrc + 63) / 64;
     p.kw = std::min(LEVEL_BLOCK_WORDS, W);
@@ -924,10 +927,10 @@ struct Evaluator {
     // part gather is 4-30 % faster at every degree but one (28000, d = 32: 2 % slower);
     // at n = 20000 it is 11-22 % faster for d <= 16 and 5 % slower for d = 32)
     p.parts = parts_default(p.kw);
-    if (p.group && p.parts && s == 1) {
+    if (p.group && p.parts && s == 1 && !getenv("ODP_ASPL")) {
       const size_t bytes = (size_t)((W + p.kw - 1) / p.kw) * 2 * n * p.kw * 8;
       size_t avail = 0, total = 0;
-      if (bytes <= SAVING_BYTES && hipMemGetInfo(&avail, &total) == hipSuccess && bytes <= avail / 2) p.group = 0;
+      if (bytes <= SAVING_BYTES && hipMemGetInfo(&avail, &total) == hipSuccess && bytes <= avail / 8) p.group = 0;
     }
     if (tile_capable()) {
       // grid graphs: 2-word blocks and temporal tiles (k_tile); MATRIX_SAVING
