@@ -2814,7 +2814,7 @@ __global__ __launch_bounds__(1024) void k_anneal(AnnealArgs a)
   extern __shared__ __attribute__((aligned(16))) u32 lds[];
   __shared__ __attribute__((aligned(16))) u32 s_part[2][16];
   __shared__ int s_mv[5], s_dec[3];
-  __shared__ AnnealState S;          // the chain's state; only wave 0 reads or writes it
+  __shared__ AnnealState S;          // the chain's state: wave 0 reads it, its lane 0 writes it
   const int tid = threadIdx.x, nth = blockDim.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   if (tid < 32 && (tid & 15) >= (nth + 63) / 64) s_part[tid >> 4][tid & 15] = 0;
@@ -2844,9 +2844,11 @@ __global__ __launch_bounds__(1024) void k_anneal(AnnealArgs a)
         anneal_swap(tab, dp, deg, x, bx, y, dy, lane);
         found = 1; ma = x; mb = bx; mc = y; md = dy;
       }
-      S.rng[0] = rng[0]; S.rng[1] = rng[1]; S.rng[2] = rng[2]; S.rng[3] = rng[3];
-      if (!found) S.stop = 1;
-      s_mv[0] = found; s_mv[1] = ma; s_mv[2] = mb; s_mv[3] = mc; s_mv[4] = md;
+      if (lane == 0) {
+        S.rng[0] = rng[0]; S.rng[1] = rng[1]; S.rng[2] = rng[2]; S.rng[3] = rng[3];
+        if (!found) S.stop = 1;
+        s_mv[0] = found; s_mv[1] = ma; s_mv[2] = mb; s_mv[3] = mc; s_mv[4] = md;
+      }
     }
     __syncthreads();
     if (!s_mv[0]) break;
@@ -2875,7 +2877,7 @@ __global__ __launch_bounds__(1024) void k_anneal(AnnealArgs a)
         }
       }
       if (abort) {
-        if (lane == 0) atomicOr(&a.st->err, 1);
+        if (lane == 0) { atomicOr(&a.st->err, 1); s_dec[2] = 1; }
       } else {
         sum = (u64)wave_sum_dpp((u32)(sum & 0xffffff)) + ((u64)wave_sum_dpp((u32)(sum >> 24)) << 24);
         diam = (u32)wave_max((int)diam);
@@ -2887,30 +2889,34 @@ __global__ __launch_bounds__(1024) void k_anneal(AnnealArgs a)
         double aspl = lsum / (((double)n - 1) * n);
         lsum /= 2.0;
         if (d > n) { d = INT_MAX; lsum = LONG_MAX; aspl = DBL_MAX; }
-        S.steps++;
+        // every lane reads the state and decides alike; lane 0 stores what changed
+        AnnealState q = S;
+        q.steps++;
         int improved = 0, accept;
-        if (d < S.best_d || (d == S.best_d && aspl < S.best_a)) {
+        if (d < q.best_d || (d == q.best_d && aspl < q.best_a)) {
           improved = 1;
-          S.best_d = d; S.best_sum = lsum; S.best_a = aspl;
-          if (d == S.low_d && aspl == S.low_a) S.optimum = 1;
+          q.best_d = d; q.best_sum = lsum; q.best_a = aspl;
+          if (d == q.low_d && aspl == q.low_a) q.optimum = 1;
         }
-        if (S.optimum) accept = 1;              // the loop ends here; the move stays
-        else if (S.hill) accept = aspl <= S.cur_a;
-        else if (d < S.cur_d && !S.prio) accept = 1;
-        else if (d > S.cur_d && !S.prio) accept = 0;
-        else if (aspl <= S.cur_a) accept = 1;
+        if (q.optimum) accept = 1;              // the loop ends here; the move stays
+        else if (q.hill) accept = aspl <= q.cur_a;
+        else if (d < q.cur_d && !q.prio) accept = 1;
+        else if (d > q.cur_d && !q.prio) accept = 0;
+        else if (aspl <= q.cur_a) accept = 1;
         else {
-          const double diff = (S.cur_a - aspl) * n * (n - 1);
-          const double u = ((double)(anneal_next(S.rng) >> 11) + 0.5) / 9007199254740992.0;
-          accept = exp(diff / S.temp) > u;
+          const double diff = (q.cur_a - aspl) * n * (n - 1);
+          const double u = ((double)(anneal_next(q.rng) >> 11) + 0.5) / 9007199254740992.0;
+          accept = exp(diff / q.temp) > u;
         }
-        if (!S.optimum) {
-          if (accept) { S.cur_d = d; S.cur_a = aspl; S.accepted++; }
-          S.temp *= S.cooling;
+        if (!q.optimum) {
+          if (accept) { q.cur_d = d; q.cur_a = aspl; q.accepted++; }
+          q.temp *= q.cooling;
         }
-        s_dec[0] = improved; s_dec[1] = accept;
+        if (lane == 0) {
+          S = q;
+          s_dec[0] = improved; s_dec[1] = accept; s_dec[2] = 2 * q.optimum;
+        }
       }
-      s_dec[2] = abort | 2 * S.optimum;
     }
     __syncthreads();
     if (s_dec[2] & 1) break;
