@@ -76,6 +76,9 @@ int  ODPX_Autotune(void *adjacency, int repeats);
 /* ---- device-resident evaluation ---------------------------------------- */
 /* Uploads adjacency to the evaluator's device copy without evaluating. */
 void ODPX_Upload_adjacency(void *adjacency);
+/* Entries of the adjacency that these calls and ODP_Set_aspl read
+ * (nodes / symmetries * degree of the active Init; 0 without one). */
+long long ODPX_Table_entries(void);
 /* Evaluates the adjacency already on the device (after ODP_Set_aspl or
  * ODPX_Upload_adjacency, and any ODPX_Swap_device since). */
 void ODPX_Set_aspl_resident(int *diameter, long *sum, double *ASPL);

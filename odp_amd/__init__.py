@@ -138,6 +138,7 @@ def load():
     _sig(lib, "ODPX_Set_plan", _I, [ctypes.POINTER(Plan)])
     _sig(lib, "ODPX_Autotune", _I, [_P, _I])
     _sig(lib, "ODPX_Upload_adjacency", None, [_P])
+    _sig(lib, "ODPX_Table_entries", ctypes.c_longlong, [])
     _sig(lib, "ODPX_Set_aspl_resident", None, [ip, ctypes.POINTER(_L), ctypes.POINTER(_D)])
     _sig(lib, "ODPX_Swap_device", _I, [_I, _I, _I, _I])
     _sig(lib, "ODPX_Set_aspl_shard", _I, [_I, _I, ctypes.POINTER(ctypes.c_longlong), ip, ip])
@@ -183,37 +184,49 @@ def _ptr(a):
 
 # ---- the ODP_* lifecycle ---------------------------------------------------
 
-class _Keep:
-    adjacency = None
+class _Init:
+    entries = 0             # of the table that the Init made here takes
+
+
+def _table(adjacency):
+    """The table as the library reads it; ValueError if it is shorter than the active Init's."""
+    a = _i32(adjacency)
+    if a.size < _Init.entries and a.size < load().ODPX_Table_entries():
+        raise ValueError(f"adjacency of {a.size} entries for an Init of {load().ODPX_Table_entries()}")
+    return a
 
 
 def init_aspl_general(nodes, degree, num_degrees=None):
     """ODP_Init_aspl_general (aspl_cuda.cu:159-162)."""
     nd = None if num_degrees is None else _i32(num_degrees)
     load().ODP_Init_aspl_general(nodes, degree, _ptr(nd))
+    _Init.entries = nodes * degree
 
 
 def init_aspl_general_s(nodes, degree, num_degrees, symmetries):
     """ODP_Init_aspl_general_s (aspl_cuda.cu:164-179); num_degrees has nodes/symmetries entries."""
     nd = None if num_degrees is None else _i32(num_degrees)
     load().ODP_Init_aspl_general_s(nodes, degree, _ptr(nd), symmetries)
+    _Init.entries = nodes // symmetries * degree
 
 
 def init_aspl_grid(width, height, degree, num_degrees=None):
     """ODP_Init_aspl_grid (aspl_cuda.cu:181-186)."""
     nd = None if num_degrees is None else _i32(num_degrees)
     load().ODP_Init_aspl_grid(width, height, degree, _ptr(nd))
+    _Init.entries = width * height * degree
 
 
 def init_aspl_grid_s(width, height, degree, num_degrees, symmetries):
     """ODP_Init_aspl_grid_s (aspl_cuda.cu:188-224)."""
     nd = None if num_degrees is None else _i32(num_degrees)
     load().ODP_Init_aspl_grid_s(width, height, degree, _ptr(nd), symmetries)
+    _Init.entries = width * height // symmetries * degree
 
 
 def set_aspl(adjacency):
     """ODP_Set_aspl (aspl_cuda.cu:242-263) -> (diameter, sum, ASPL)."""
-    a = _i32(adjacency)
+    a = _table(adjacency)
     d, s, x = ctypes.c_int(), ctypes.c_long(), ctypes.c_double()
     load().ODP_Set_aspl(_ptr(a), ctypes.byref(d), ctypes.byref(s), ctypes.byref(x))
     return d.value, s.value, x.value
@@ -225,7 +238,7 @@ def finalize_aspl():
 
 
 def upload_adjacency(adjacency):
-    a = _i32(adjacency)
+    a = _table(adjacency)
     load().ODPX_Upload_adjacency(_ptr(a))
 
 
@@ -283,7 +296,7 @@ def set_plan(**kw):
 
 
 def autotune(adjacency, repeats=2):
-    a = _i32(adjacency)
+    a = _table(adjacency)
     return load().ODPX_Autotune(_ptr(a), repeats)
 
 
@@ -478,7 +491,7 @@ def restore_grid(r, adjacency):
 
 def anneal(adjacency, ncalcs, max_temp=100.0, min_temp=0.217147, hill_climbing=False, aspl_priority=False, seed=1):
     """ODPX_Anneal on the active general Init: returns (best adjacency, result dict)."""
-    a = np.array(adjacency, dtype=np.int32, order="C", copy=True)
+    a = np.array(_table(adjacency), copy=True)
     r = AnnealResult()
     if load().ODPX_Anneal(_ptr(a), int(ncalcs), float(max_temp), float(min_temp), int(bool(hill_climbing)),
                           int(bool(aspl_priority)), int(seed), ctypes.byref(r)) != 0:

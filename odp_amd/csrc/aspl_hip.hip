@@ -2230,6 +2230,11 @@ extern "C" int ODPX_Get_plan(ODPX_Plan* p)
   return 0;
 }
 
+extern "C" long long ODPX_Table_entries(void)
+{
+  return E.active ? (long long)E.ev.adj_elems() : 0;
+}
+
 extern "C" int ODPX_Set_plan(const ODPX_Plan* p)
 {
   RandFence rand_fence;
