@@ -1098,8 +1098,8 @@ struct Evaluator {
       }
       // persistent grid: every workgroup the CUs hold at once, a multiple of the XCD count
       int occ = 0, occ_ls = 0;
-      HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_pgather<false, true>, PG_WG, 0));
-      HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ_ls, k_pgather<true, true>, PG_WG, 0));
+      HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_pgather<false, true, true>, PG_WG, 0));
+      HIPC(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ_ls, k_pgather<true, true, true>, PG_WG, 0));
       occ = std::max(1, std::min(occ, occ_ls));
       r.pgrid = ODP_NXCD * std::max(1, C.ncu / ODP_NXCD) * occ;
       // folded levels need the whole matrix resident, a task per PG_UNIT rows
@@ -1413,8 +1413,10 @@ struct Evaluator {
       a.cut_full = r.cut_full; a.cut_fold = r.cut_fold;
       const bool ls = (mode & LV_LIST) != 0;
       const bool nt = pg_streamed() != 0;
-      auto kern = ls ? (nt ? k_pgather<true, true> : k_pgather<true, false>)
-                     : (nt ? k_pgather<false, true> : k_pgather<false, false>);
+      auto kern = asym ? (ls ? (nt ? k_pgather<true, true, true> : k_pgather<true, false, true>)
+                             : (nt ? k_pgather<false, true, true> : k_pgather<false, false, true>))
+                       : (ls ? (nt ? k_pgather<true, true, false> : k_pgather<true, false, false>)
+                             : (nt ? k_pgather<false, true, false> : k_pgather<false, false, false>));
       hipLaunchKernelGGL(kern, dim3(r.pgrid), dim3(PG_WG), 0, st, r.tasks + lv.first, L, RING, mode, lst, a);
     } else {
       const bool ls = (mode & LV_LIST) != 0;

@@ -911,7 +911,7 @@ __device__ __forceinline__ void row_store(u64v2 o, u64v2* p)
 // are cut into pieces of their rows (2^cut of them) dealt over the workgroups.
 // The gathers are buffer loads bounded by the slab (out-of-range offsets read
 // zero).  LS: listing; NT: rows streamed past the caches.
-template <bool LS, bool NT>
+template <bool LS, bool NT, bool FOLD>
 __global__ __launch_bounds__(PG_WG) void k_pgather(const LevelTask* __restrict__ tasks, int level, int ring,
                                                    int mode, LvList lst, PgArgs a)
 {
@@ -925,7 +925,7 @@ __global__ __launch_bounds__(PG_WG) void k_pgather(const LevelTask* __restrict__
   static_assert(PG_UNIT / (PG_WG / 64) == 64, "a wave stores and transposes 64 rows of a unit");
   const bool count = (mode & LV_COUNT) != 0, store = (mode & LV_STORE) != 0;
   const int w = 2 * (lane & 7);                       // the lane's two words of a row
-  const bool fold = a.asym && __builtin_amdgcn_readfirstlane(*a.asym) == 0;
+  const bool fold = FOLD && __builtin_amdgcn_readfirstlane(*a.asym) == 0;
   if (fold) {
     // a unit stands for two blocks, so all run until none has to
     bool run = false;
