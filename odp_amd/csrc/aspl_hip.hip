@@ -964,9 +964,9 @@ struct Evaluator {
   // ---- direct enumeration of the first levels (k_direct) ----
   // gather levels run k_pgather: a plan with parts, plain (not frontier, not tile) levels
   bool pg_on() const { return plan.plan == ODPX_PLAN_LEVEL && lr.parts > 0 && !lv.fr && !lv.tk; }
-  // k_direct reads the 16-bit table when it exists with the 32-bit table's width
   // whether the gather levels' rows are streamed: the resident blocks' two buffers pass the last-level cache
   int pg_streamed() const { return (size_t)lr.group * 2 * n * lr.kwp * 8 > MALL_BYTES ? 1 : 0; }
+  // k_direct reads the 16-bit table when it exists with the 32-bit table's width
   bool direct16() const
   {
     return plan.plan == ODPX_PLAN_LEVEL && lr.direct > 0 && d_nbr16 && dp16 == dpad;
@@ -1080,10 +1080,9 @@ struct Evaluator {
       dfree(&r.wgm); dalloc(&r.wgm, wbytes); r.wgm_bytes = wbytes;
       HIPC(hipMemset(r.wgm, 0, wbytes));
     }
-    // the XCD-phased gather applies to 16-word rows and runs of at most 63 ids
+    r.fold = false;
     // the XCD-phased gather applies to 16-word rows, runs of at most 63 ids and
     // ids below 2^22 (the pair lists pack the row in the unit beside the id)
-    r.fold = false;
     r.parts = (plan.parts > 0 && kwp == 16 && dpad + 1 <= 63 && n <= (1 << 22)) ? plan.parts : 0;
     plan.parts = r.parts;              // the plan reports what runs
     if (r.parts) {
@@ -1438,8 +1437,9 @@ struct Evaluator {
   // Neighbours the level before the next evaluation's last one should take: with
   // a share p of the pairs missing before it, a chunk of 128 is unsaturated after
   // k neighbours with probability about 128 p^k (what the row itself holds, its
-  // neighbours mostly hold too).  All of them: the level still stores nothing.  Zero when the level leaves too many
-  // pairs for k_thin2's two-step reads.
+  // neighbours mostly hold too).  More than a row has: it takes them all and still
+  // stores nothing.  Zero when the level leaves too many pairs for k_thin2's
+  // two-step reads.
   int thin_choice() const
   {
     const int L = lv.lmax - 1;
@@ -2918,11 +2918,10 @@ static void balance_env(int* banks, int* group)
   *banks = b; *group = g;
 }
 
-// the resident launch's task table under the current policy: per graph the
-// widest block its size class allows, longest blocks first (short queue tail)
-// the task table: per chunk the widest blocks first, then each width's blocks
-// longest first (short queue tails).  A graph's blocks cost the same, so the
-// graphs are sorted, not the blocks.
+// the resident launches' task table under the current policy (per graph the
+// widest block its size class allows): per chunk the widest blocks first, then
+// each width's blocks longest first (short queue tails).  A graph's blocks cost
+// the same, so the graphs are sorted, not the blocks.
 static void batch_build_tasks()
 {
   batch_drop_graph();

@@ -659,7 +659,9 @@ struct PgArgs {
 // grouped by part with the part offsets.  A part's thin pairs come first: the
 // row itself and its first `thin` neighbours, in the order of the parts (a thin
 // level, LV_THIN, takes those alone); rows ascend within either group.
-// DMAX >= dpad + 1 bounds the ids a row holds in registers.
+// DMAX >= dpad + 1 bounds the ids a row holds in registers (DMAX = 64: 22 of 150
+// spilled since the pairs have a thin part, 92 bytes a lane; with the levels it
+// serves, a move and an evaluation of n = 50000, d = 60 went 2563 -> 1463 us).
 //
 // A device swap (or a small change of an uploaded table) hands the changed
 // entries to the units it rebuilds (rows, positions in the row, old and new
@@ -910,7 +912,10 @@ __device__ __forceinline__ void row_store(u64v2 o, u64v2* p)
 // multiple of 8 works.  The units of the last round, when they do not fill it,
 // are cut into pieces of their rows (2^cut of them) dealt over the workgroups.
 // The gathers are buffer loads bounded by the slab (out-of-range offsets read
-// zero).  LS: listing; NT: rows streamed past the caches.
+// zero).  LS: listing; NT: rows streamed past the caches; FOLD: folds where the
+// table is symmetric (128 registers, four more spilled to 20 bytes a lane; the
+// others, for launches that never fold, 111 without a spill: general_s n = 100000,
+// d = 6, s = 2 3190 -> 3084 us a call).
 template <bool LS, bool NT, bool FOLD>
 __global__ __launch_bounds__(PG_WG) void k_pgather(const LevelTask* __restrict__ tasks, int level, int ring,
                                                    int mode, LvList lst, PgArgs a)
@@ -1472,7 +1477,7 @@ __global__ __launch_bounds__(LEVEL_WG) void k_thin2(const LevelTask* __restrict_
     const int* __restrict__ nbr = T.nbr;
     const int dp = T.dpad, m = dp * (dp + 1);
     u64x2 x = x0;
-    for (int i0 = lane; i0 < m; i0 += 64 * 4) {       // four pairs a lane in flight (past the last: the chunk's own row)
+    for (int i0 = lane; i0 < m; i0 += 64 * 4) {       // four pairs a lane in flight (past the last: the first neighbour's row, which counts anyway)
       int u[4], q[4], v[4];
 #pragma unroll
       for (int c = 0; c < 4; c++) {
@@ -1655,6 +1660,8 @@ __global__ void k_tile_plan(const LevelTask* __restrict__ tasks, int ntasks, int
 // unit was loaded, written back or waited at a barrier, 16 us a unit against the
 // 8 its reads take.  256 x 256 grid, d = 8: 144 -> 122 us a launch, 118 with the
 // offsets of cells outside a level's window read from one row and the gains added between lanes.
+// (The instance for 8 ids spills five registers, 24 bytes a lane, at the 128 that
+// two workgroups a CU leave it; the two-copy one of 99 had none.)
 
 // cell (lx, ly) of the region of a tile: thread tid owns (wave + waves m, lane),
 // a wave whole region columns
@@ -1781,16 +1788,16 @@ __global__ __launch_bounds__(TILE_THREADS(DP), 4) void k_tile(const LevelTask* _
           if (!(o.x == f0 && o.y == f1)) {
             const u32* w = off[ONE ? m & 1 : m];
 #pragma unroll
-          for (int j = 0; j < DP / 2; j++) {
-            // the window keeps every neighbour inside the region: a cell at least
-            // (i + 1) lmax from its edges, and no offset longer than lmax cells
-            // (k_tgeom flags longer ones, which end the run)
-            const int s0 = sl + (int)(short)(w[j] & 0xffff);
-            const int s1 = sl + (int)(short)(w[j] >> 16);
-            const u64x2 a = src[s0], c = src[s1];
-            x.x |= a.x | c.x;
-            x.y |= a.y | c.y;
-          }
+            for (int j = 0; j < DP / 2; j++) {
+              // the window keeps every neighbour inside the region: a cell at least
+              // (i + 1) lmax from its edges, and no offset longer than lmax cells
+              // (k_tgeom flags longer ones, which end the run)
+              const int s0 = sl + (int)(short)(w[j] & 0xffff);
+              const int s1 = sl + (int)(short)(w[j] >> 16);
+              const u64x2 a = src[s0], c = src[s1];
+              x.x |= a.x | c.x;
+              x.y |= a.y | c.y;
+            }
           }
           if (ONE) nx[ONE ? m : 0] = x;
           else dst[sl] = x;
