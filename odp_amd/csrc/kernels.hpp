@@ -2899,7 +2899,7 @@ __global__ __launch_bounds__(1024) void k_anneal(AnnealArgs a)
         // every lane reads the state and decides alike; lane 0 stores what changed
         AnnealState q = S;
         q.steps++;
-        int improved = 0, accept;
+        int improved = 0, accept, drawn = 0;
         if (d < q.best_d || (d == q.best_d && aspl < q.best_a)) {
           improved = 1;
           q.best_d = d; q.best_sum = lsum; q.best_a = aspl;
@@ -2914,13 +2914,17 @@ __global__ __launch_bounds__(1024) void k_anneal(AnnealArgs a)
           const double diff = (q.cur_a - aspl) * n * (n - 1);
           const double u = ((double)(anneal_next(q.rng) >> 11) + 0.5) / 9007199254740992.0;
           accept = exp(diff / q.temp) > u;
+          drawn = 1;
         }
         if (!q.optimum) {
           if (accept) { q.cur_d = d; q.cur_a = aspl; q.accepted++; }
           q.temp *= q.cooling;
         }
         if (lane == 0) {
-          S = q;
+          S.steps = q.steps; S.temp = q.temp; S.optimum = q.optimum;
+          if (improved) { S.best_d = q.best_d; S.best_sum = q.best_sum; S.best_a = q.best_a; }
+          if (accept) { S.cur_d = q.cur_d; S.cur_a = q.cur_a; S.accepted = q.accepted; }
+          if (drawn) for (int i = 0; i < 4; i++) S.rng[i] = q.rng[i];
           s_dec[0] = improved; s_dec[1] = accept; s_dec[2] = 2 * q.optimum;
         }
       }
