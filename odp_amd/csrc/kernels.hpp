@@ -2123,14 +2123,15 @@ struct ResTask {
 // walks stay below a pulled level's row reads (cost 1: measured best for the
 // 1024-graph batch, 20.2 ms against 20.3 at 2, 20.55 at 4, 20.5 at 0.5).
 // Returns the first pulled level (1: level 0 alone, whose l * (deg + 1) walks
-// of at most one step always beat reading the table).
+// of at most one step always beat reading the table).  A level's prefixes
+// (l * deg^L) stay below 2^24 whatever the cost: res_run's FastDiv decodes them.
 __host__ __device__ inline int res_walk_levels(int n, int deg, int l, double cost = 1.0)
 {
   int K = 1;
   double w = (double)l * deg;                        // walks of one step
   for (int L = 1; L < 8; L++) {
     w *= deg;                                        // walks of L + 1 steps
-    if (w * cost * (L + 1) > (double)n * (deg + 1)) break;
+    if (w * cost * (L + 1) > (double)n * (deg + 1) || w >= 16777216.0 * deg) break;
     K = L + 1;
   }
   return K;
